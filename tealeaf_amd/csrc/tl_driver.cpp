@@ -24,6 +24,7 @@
 
 #include "tealeaf_hip.h"
 #include "tl_adjoint.h"
+#include "tl_chip.h"
 #include "tl_loop.h"
 #include "tl_mixed.h"
 
@@ -159,6 +160,7 @@ struct tlhip_problem {
     // (tlhip2d_cg_calc_pw); flush_p() applies it where p is read otherwise.
     bool pending_p = false;
     double pending_beta = 0.0;
+    tl::chip::Plan chip;         // tiles of the one-launch loops; ok where the grid fits
 
     // -------------------------------------------------------- kernels
     int local_halos(int depth)
@@ -349,8 +351,28 @@ struct tlhip_problem {
         return rc;
     }
 
+    // CG steps of grids that fit the chip run many to a launch (tl_chip.h).
+    // The host-driven loop launches one at a time: the same bits.
+    bool chip_cg() const { return chip.ok && g_cg_cond && g_cg_fusion && interior(); }
+
+    int cg_step_chip(int tt, double* rro, double* error)
+    {
+        tl::loop::StopRule never{};
+        tl::chip::Outcome o;
+        TRY(tl::loop::begin(*rro, s.max_iters));
+        tl::loop::end();
+        never.eps = -1.0;
+        TRY(tl::chip::cg(chip, u, p, r, kx, ky, kz, tt, 1, never, &o));
+        cg_alphas[tt] = o.alpha;
+        cg_betas[tt] = o.beta;
+        *rro = *error = o.rep.rrn;
+        rep->n_cg_steps++;
+        return 0;
+    }
+
     int cg_main_step(int tt, double* rro, double* error)
     {
+        if (chip_cg()) return cg_step_chip(tt, rro, error);
         double alpha = 0.0, rrn = 0.0;
         if (cond_ok()) {
             TRY(cg_step_cond(rro, &alpha, &rrn));
@@ -777,6 +799,30 @@ struct tlhip_problem {
         return 0;
     }
 
+    // cg_resident's run from t0 with all its iterations in one launch (a long
+    // run: a few thousand per launch).
+    int cg_run_chip(int t0, int sw, double* rro, double* error, int* last, tl::loop::Report* rp)
+    {
+        if (t0 < 0 || t0 >= s.max_iters)
+            return tl_fail(TLHIP_ERR_ARG, "resident loop: no iteration to run from %d", t0);
+        TRY(tl::loop::begin(*rro, s.max_iters));
+        tl::loop::end();
+        const tl::loop::StopRule rule = stop_rule(sw);
+        tl::chip::Outcome o{};
+        for (int from = t0;; from = o.last + 1) {
+            TRY(tl::chip::cg(chip, u, p, r, kx, ky, kz, from, s.max_iters - from, rule, &o));
+            TRY(check_report(o.rep, o.last, sw));
+            if (o.rep.flags || o.last + 1 >= s.max_iters) break;
+        }
+        TRY(halo_update(1));
+        TRY(tl::loop::logs(t0, o.last - t0 + 1, &cg_alphas[t0], &cg_betas[t0]));
+        *last = o.last;
+        *rp = o.rep;
+        *rro = o.rep.rrn;
+        *error = o.rep.err;
+        return 0;
+    }
+
     // CG iterations from t0 until the stop test passes (*done, *tt = that
     // iteration), the switch test of the next iteration passes (*tt = the
     // last CG iteration), or max_iters - 1 has run (*tt = max_iters - 1).
@@ -785,9 +831,12 @@ struct tlhip_problem {
         for (int from = t0;;) {
             int last;
             tl::loop::Report rp;
-            TRY(run_resident(from, sw, true,
-                             [&](const tl::loop::StopRule& rule, int) { return cg_body(rule); }, rro,
-                             error, &last, &rp, true, can_defer_p() || cond3_ok()));
+            if (chip_cg())
+                TRY(cg_run_chip(from, sw, rro, error, &last, &rp));
+            else
+                TRY(run_resident(from, sw, true,
+                                 [&](const tl::loop::StopRule& rule, int) { return cg_body(rule); },
+                                 rro, error, &last, &rp, true, can_defer_p() || cond3_ok()));
             rep->n_cg_steps += last - from + 1;
             *tt = last;
             TRY(confirm(rp, done));
@@ -1754,6 +1803,7 @@ void alloc_partners(tlhip_problem* P, int* rc)
     // partner of p: the fused calc_p + calc_w (2D; 3D with cond) and the
     // 2D fused Chebyshev loop
     if (P->dims == 2 || cg) P->p_alt = dalloc(P->n, rc);
+    P->chip = tl::chip::plan(P->dims, P->x, P->y, P->z, P->hd);
     // partner of r: the fused PPCG inner loops (2D ring, 3D two-step launch)
     if (P->s.solver == 3) P->r_alt = dalloc(P->n, rc);
 }

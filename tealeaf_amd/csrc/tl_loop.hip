@@ -374,6 +374,12 @@ int logs(int j0, int n, double* alphas, double* betas)
     return 0;
 }
 
+void log_ptrs(double** alphas, double** betas)
+{
+    *alphas = g_loop.alog;
+    *betas = g_loop.blog;
+}
+
 void release()
 {
     Host& h = g_loop;

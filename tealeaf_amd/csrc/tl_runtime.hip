@@ -6,6 +6,7 @@
 // rank, 2d/drivers/*_driver.c call run_* one after another), and so is this
 // runtime: calls from several host threads at once are not supported.
 #include "tl_ops.h"
+#include "tl_chip.h"
 #include "tl_loop.h"
 #include "tealeaf_hip.h"
 
@@ -206,6 +207,7 @@ extern "C" int tlhip_finalise(void)
     if (!g_rt.initialised) return 0;
     // Teardown: report the first failure but release everything regardless.
     hipError_t first = hipStreamSynchronize(g_rt.stream);
+    tl::chip::release();
     tl::loop::release();
     hipError_t e[6] = {hipFree(g_rt.red.partials), hipSuccess,
                        hipFree(g_rt.red.result), hipHostFree(g_rt.red.mailbox),
