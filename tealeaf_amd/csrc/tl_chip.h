@@ -36,7 +36,7 @@ struct Outcome {
 // CG iterations it0, it0 + 1, ... of r, p and u (in place, r and p of the
 // state before it0): at most `count`, fewer when `rule` fires.  p has the
 // last iteration's calc_p applied; halos are not touched.  alpha and beta of
-// every iteration go to the loop's logs (loop::begin has been called).
+// every iteration go to the loop's logs (loop::reserve_logs has been called).
 int cg(const Plan& pl, double* u, double* p, double* r, const double* kx, const double* ky,
        const double* kz, int it0, int count, const loop::StopRule& rule, Outcome* out);
 

@@ -716,7 +716,7 @@ int with_plan(const Plan& pl, F&& f)
     return pl.dims == 2 ? cells(Int<2>{}) : cells(Int<3>{});
 }
 
-int prepare(size_t xdoubles, const char* what)
+int prepare(int nb, size_t xdoubles, const char* what)
 {
     Host& h = g_chip;
     TL_TRY(tl_ensure_init());
@@ -733,6 +733,7 @@ int prepare(size_t xdoubles, const char* what)
         CHIP_HIP(hipMalloc(&h.xbuf, sizeof(double) * xdoubles), what);
         h.xlen = xdoubles;
     }
+    if (nb == 1) return 0;        // a single block has nobody to meet
     const int n = kPhases * kMaxBlocks * kSums;
     hipLaunchKernelGGL(k_empty, dim3((n + 255) / 256), dim3(256), 0, tl_stream(), h.slots, n);
     return tl_check_launch(what);
@@ -846,7 +847,7 @@ int cg(const Plan& pl, double* u, double* p, double* r, const double* kx, const 
         constexpr int LXS = decltype(row)::value;
         const Geo g = geo_of(pl);
         const int nb = pl.blocks();
-        TL_TRY(prepare(2 * (size_t)nb * faces_of<D, K>(pl.lxs).total(), what));
+        TL_TRY(prepare(nb, 2 * (size_t)nb * faces_of<D, K>(pl.lxs).total(), what));
         const size_t lds = lds_bytes<D, K>(pl.lxs);
         const void* fn = (const void*)k_chip_cg<D, K, LXS>;
         CHIP_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), what);

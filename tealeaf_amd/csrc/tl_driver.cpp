@@ -230,11 +230,13 @@ struct tlhip_problem {
         rz = rz_;
         if (dims == 2) {
             TRY(tlhip2d_cg_init(x, y, hd, s.coefficient, rx, ry, rro, density, energy, u, p, r, w, kx, ky));
-            if (cond_ok()) TRY(tlhip2d_cg_cond(x, y, hd, s.coefficient, density, cond));
+            if (cond_ok() && !(chip_cg() && s.solver != 3))
+                TRY(tlhip2d_cg_cond(x, y, hd, s.coefficient, density, cond));
         } else {
             TRY(tlhip3d_cg_solver_init(x, y, z, hd, s.coefficient, rx, ry, rz, rro, density,
                                        energy, u, p, r, w, kx, ky, kz));
-            if (cond3_ok()) TRY(tlhip3d_cg_cond(x, y, z, hd, s.coefficient, density, cond));
+            if (cond3_ok() && !chip_cg())
+                TRY(tlhip3d_cg_cond(x, y, z, hd, s.coefficient, density, cond));
         }
         reset_fields();
         fields[F_U] = fields[F_P] = true;
@@ -359,8 +361,7 @@ struct tlhip_problem {
     {
         tl::loop::StopRule never{};
         tl::chip::Outcome o;
-        TRY(tl::loop::begin(*rro, s.max_iters));
-        tl::loop::end();
+        TRY(tl::loop::reserve_logs(s.max_iters));
         never.eps = -1.0;
         TRY(tl::chip::cg(chip, u, p, r, kx, ky, kz, tt, 1, never, &o));
         cg_alphas[tt] = o.alpha;
@@ -805,8 +806,7 @@ struct tlhip_problem {
     {
         if (t0 < 0 || t0 >= s.max_iters)
             return tl_fail(TLHIP_ERR_ARG, "resident loop: no iteration to run from %d", t0);
-        TRY(tl::loop::begin(*rro, s.max_iters));
-        tl::loop::end();
+        TRY(tl::loop::reserve_logs(s.max_iters));
         const tl::loop::StopRule rule = stop_rule(sw);
         tl::chip::Outcome o{};
         for (int from = t0;; from = o.last + 1) {
@@ -815,7 +815,9 @@ struct tlhip_problem {
             if (o.rep.flags || o.last + 1 >= s.max_iters) break;
         }
         TRY(halo_update(1));
-        TRY(tl::loop::logs(t0, o.last - t0 + 1, &cg_alphas[t0], &cg_betas[t0]));
+        // (read by the eigenvalue estimate only)
+        if (s.solver != 1)
+            TRY(tl::loop::logs(t0, o.last - t0 + 1, &cg_alphas[t0], &cg_betas[t0]));
         *last = o.last;
         *rp = o.rep;
         *rro = o.rep.rrn;
@@ -849,23 +851,28 @@ struct tlhip_problem {
     {
         double rro;
         TRY(cg_init_driver(rx, ry, rz, &rro));
-        int tt = 0;
+        return cg_loop(&rro, error, &rep->printed_cg_iters);
+    }
+
+    // CG from the r = p in hand until the stop test passes or max_iters
+    // iterations have run; *tt as cg_driver.c prints it.
+    int cg_loop(double* rro, double* error, int* tt)
+    {
+        *tt = 0;
         if (resident_cg() && s.max_iters > 0) {
             bool done;
-            TRY(cg_resident(0, 0, &rro, error, &tt, &done));
-            if (!done) tt = s.max_iters;
+            TRY(cg_resident(0, 0, rro, error, tt, &done));
+            if (!done) *tt = s.max_iters;
         } else {
-            for (tt = 0; tt < s.max_iters; ++tt) {
-                TRY(cg_main_step(tt, &rro, error));
+            for (; *tt < s.max_iters; ++*tt) {
+                TRY(cg_main_step(*tt, rro, error));
                 TRY(halo_update(1));
                 bool done;
                 TRY(stop(error, &done));
                 if (done) break;
             }
         }
-        TRY(flush_p());
-        rep->printed_cg_iters = tt;
-        return 0;
+        return flush_p();
     }
 
     bool switch_now(int started, int tt, double error) const
@@ -1520,16 +1527,7 @@ struct tlhip_problem {
         TRY(norm2(r, &rro));
         TRY(start_solve());
         double error = rro;
-        int tt;
-        for (tt = 0; tt < s.max_iters; ++tt) {
-            TRY(cg_main_step(tt, &rro, &error));
-            TRY(halo_update(1));
-            bool done;
-            TRY(stop(&error, &done));
-            if (done) break;
-        }
-        TRY(flush_p());
-        report->printed_cg_iters = tt;
+        TRY(cg_loop(&rro, &error, &report->printed_cg_iters));
         report->error = error;
         return 0;
     }

@@ -68,6 +68,9 @@ int finish_err(unsigned nblocks, ErrMode mode, const StopRule& rule, const char*
 int wait(int j, Report* out);
 // alpha and beta of iterations j0 .. j0+n-1 into host arrays.
 int logs(int j0, int n, double* alphas, double* betas);
+// Make the alpha and beta logs hold at least `max_iters` entries (begin()
+// does this too).
+int reserve_logs(int max_iters);
 // Device arrays of the alpha and beta logs (for a kernel that runs whole
 // iterations itself).
 void log_ptrs(double** alphas, double** betas);

@@ -163,6 +163,19 @@ int begin(double rro, int max_iters)
                                hipHostMallocMapped | hipHostMallocCoherent), what);
         for (int i = 0; i < kRing; ++i) h.ring[i] = Slot{};
     }
+    TL_TRY(reserve_logs(max_iters));
+    hipLaunchKernelGGL(k_loop_begin, dim3(1), dim3(64), 0, tl_stream(), h.st, rro);
+    TL_TRY(tl_check_launch(what));
+    h.active = true;
+    h.iter = 0;
+    return 0;
+}
+
+int reserve_logs(int max_iters)
+{
+    const char* what = "tl::loop::reserve_logs";
+    TL_TRY(tl_ensure_init());
+    Host& h = g_loop;
     const int need = max_iters > 1 ? max_iters : 1;
     if (need > h.cap) {
         LOOP_HIP(hipStreamSynchronize(tl_stream()), what);
@@ -174,10 +187,6 @@ int begin(double rro, int max_iters)
         LOOP_HIP(hipMalloc(&h.blog, sizeof(double) * need), what);
         h.cap = need;
     }
-    hipLaunchKernelGGL(k_loop_begin, dim3(1), dim3(64), 0, tl_stream(), h.st, rro);
-    TL_TRY(tl_check_launch(what));
-    h.active = true;
-    h.iter = 0;
     return 0;
 }
 
