@@ -44,6 +44,7 @@ BYTES_PER_CELL = {
     "tlhip2d_cg_calc_pw_cond": 40,        # read p, r, cond; write p', w
     "tlhip2d_cg_calc_pw_cond.no_w": 32,   # read p, r, cond; write p' (w kept in registers)
     "tlhip2d_cg_calc_ur_cond": 48,        # read u, p, r, cond; write u, r
+    "tl_cg_pass2d": 56,                   # read u, r, p, cond; write u, r, p (a whole CG step)
     "tlhip2d_cg_calc_w": 32,              # read p, kx, ky; write w
     "tlhip2d_cg_calc_ur": 48,             # read u, p, r, w; write u, r
     "tlhip2d_cg_calc_p": 24,              # read p, r; write p
@@ -126,13 +127,12 @@ def gpu_run(args):
     # Each timed launch adds two event records to the stream (about 4% of a
     # CG iteration), so: the fused PPCG launch (the kernel with the most time)
     # and PPCG's calc_pw in the PPCG leg, the fused Chebyshev launch and the
-    # CG pair in the Chebyshev leg (its 1559 CG iterations; the same kernels
-    # at the same size run every CG iteration of all three legs), nothing
+    # CG pass in the Chebyshev leg (its 1559 CG iterations; the same kernel
+    # at the same size runs every CG iteration of all three legs), nothing
     # in the CG leg; the small rest (2-norms, finishers, halo and ring
     # copies) untimed.
     own = {"cg": [],
-           "cheby": ["tlhip2d_cheby_iterations", "tlhip2d_cg_calc_pw_cond.no_w",
-                     "tlhip2d_cg_calc_ur_cond"],
+           "cheby": ["tlhip2d_cheby_iterations", "tl_cg_pass2d"],
            "ppcg": [dominant(args), "tlhip2d_cg_calc_pw_cond"]}
     for s in solvers:
         timed = own[s]

@@ -24,6 +24,7 @@
 
 #include "tealeaf_hip.h"
 #include "tl_adjoint.h"
+#include "tl_cg_pass.h"
 #include "tl_chip.h"
 #include "tl_loop.h"
 #include "tl_mixed.h"
@@ -160,6 +161,10 @@ struct tlhip_problem {
     // (tlhip2d_cg_calc_pw); flush_p() applies it where p is read otherwise.
     bool pending_p = false;
     double pending_beta = 0.0;
+    // Sums of the r and p in hand (host-driven CG passes); formed again after
+    // anything else touched them.
+    bool have_sums = false;
+    double sums[4] = {};
     tl::chip::Plan chip;         // tiles of the one-launch loops; ok where the grid fits
 
     // -------------------------------------------------------- kernels
@@ -371,9 +376,64 @@ struct tlhip_problem {
         return 0;
     }
 
+    // 2D CG steps of larger grids: one pass per iteration (tl_cg_pass.h).
+    bool pass_cg() const { return !chip_cg() && cond_ok() && r_alt; }
+
+    int cg_pass(bool update, double alpha, double beta, double out[4])
+    {
+        TRY(tl::pass::step2d(x, y, hd, update, alpha, beta, u, r, r_alt, p, p_alt, cond, rx, ry,
+                             out));
+        if (update) {
+            std::swap(r, r_alt);
+            std::swap(p, p_alt);
+        }
+        return 0;
+    }
+
+    int need_sums()
+    {
+        if (!have_sums) TRY(cg_pass(false, 0.0, 0.0, sums));
+        have_sums = true;
+        return 0;
+    }
+
+    int cg_step_pass(int tt, double* rro, double* error)
+    {
+        TRY(need_sums());
+        double alpha, beta, rrn = 0.0;
+        if (tl::pass::scalars(sums, &alpha, &beta)) {
+            const double old = sums[tl::pass::kRR];
+            TRY(cg_pass(true, alpha, beta, sums));
+            rrn = sums[tl::pass::kRR];
+            beta = rrn / old;
+        } else {
+            // the prediction cancels: two sums, a pass apart
+            double old = sums[tl::pass::kRR];
+            have_sums = false;
+            TRY(cg_step_cond(&old, &alpha, &rrn));
+            beta = rrn / old;
+            TRY(calc_p(beta));
+        }
+        cg_alphas[tt] = alpha;
+        cg_betas[tt] = beta;
+        *rro = *error = rrn;
+        rep->n_cg_steps++;
+        return 0;
+    }
+
+    int cg_body_pass(const tl::loop::StopRule& rule, int j, int first)
+    {
+        if (j == first) TRY(tl::loop::start_pass(j, sums));
+        TRY(tl::loop2d::cg_pass(x, y, hd, u, r, r_alt, p, p_alt, cond, rx, ry, rule));
+        std::swap(r, r_alt);
+        std::swap(p, p_alt);
+        return 0;              // p is mirrored, u read pointwise: halo at the end
+    }
+
     int cg_main_step(int tt, double* rro, double* error)
     {
         if (chip_cg()) return cg_step_chip(tt, rro, error);
+        if (pass_cg()) return cg_step_pass(tt, rro, error);
         double alpha = 0.0, rrn = 0.0;
         if (cond_ok()) {
             TRY(cg_step_cond(rro, &alpha, &rrn));
@@ -443,6 +503,7 @@ struct tlhip_problem {
     int start_solve()
     {
         bb = 0.0;
+        have_sums = false;
         if (rel_tol > 0.0 || precision == 1) TRY(norm2(u0, &bb));
         return 0;
     }
@@ -486,7 +547,7 @@ struct tlhip_problem {
         if (conv) want |= tl::loop::kConverged;
         if (sw && switch_now(0, j + 1, err)) want |= tl::loop::kSwitch;
         const bool same_err = err == rp.err || (err != err && rp.err != rp.err);
-        if (want != rp.flags || !same_err)
+        if (want != (rp.flags & ~tl::loop::kCancel) || !same_err)
             return tl_fail(TLHIP_ERR_SOLVER,
                            "resident loop: device report of iteration %d differs from the host's "
                            "test (flags %d, host %d)", j, rp.flags, want);
@@ -832,13 +893,29 @@ struct tlhip_problem {
     {
         for (int from = t0;;) {
             int last;
-            tl::loop::Report rp;
+            tl::loop::Report rp{};
+            if (pass_cg()) {
+                TRY(need_sums());
+                double a, b;
+                if (!tl::pass::scalars(sums, &a, &b)) {
+                    TRY(cg_step_pass(from, rro, error));
+                    TRY(halo_update(1));
+                    TRY(stop(error, done));
+                    *tt = from++;
+                    if (*done || from >= s.max_iters || (sw && switch_now(0, from, *error))) return 0;
+                    continue;
+                }
+            }
             if (chip_cg())
                 TRY(cg_run_chip(from, sw, rro, error, &last, &rp));
             else
                 TRY(run_resident(from, sw, true,
-                                 [&](const tl::loop::StopRule& rule, int) { return cg_body(rule); },
+                                 [&](const tl::loop::StopRule& rule, int j) {
+                                     return pass_cg() ? cg_body_pass(rule, j, from)
+                                                      : cg_body(rule);
+                                 },
                                  rro, error, &last, &rp, true, can_defer_p() || cond3_ok()));
+            have_sums = false;
             rep->n_cg_steps += last - from + 1;
             *tt = last;
             TRY(confirm(rp, done));
@@ -1803,7 +1880,9 @@ void alloc_partners(tlhip_problem* P, int* rc)
     if (P->dims == 2 || cg) P->p_alt = dalloc(P->n, rc);
     P->chip = tl::chip::plan(P->dims, P->x, P->y, P->z, P->hd);
     // partner of r: the fused PPCG inner loops (2D ring, 3D two-step launch)
-    if (P->s.solver == 3) P->r_alt = dalloc(P->n, rc);
+    // and the 2D CG passes
+    if (P->s.solver == 3 || (P->dims == 2 && cg && !P->chip.ok && P->x % 2 == 0))
+        P->r_alt = dalloc(P->n, rc);
 }
 }  // namespace
 

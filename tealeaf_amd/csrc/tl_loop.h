@@ -34,11 +34,13 @@ struct StopRule {
     int presteps;
 };
 
-enum : int { kConverged = 1, kSwitch = 2 };
+// kCancel: a CG pass's prediction cancels (tl_cg_pass.h); the host runs the
+// next iteration itself.
+enum : int { kConverged = 1, kSwitch = 2, kCancel = 4 };
 
 struct Report {
     double rrn, err;
-    int flags;           // kConverged | kSwitch
+    int flags;           // kConverged | kSwitch | kCancel
 };
 
 constexpr int kAhead = 4;   // iterations in flight beyond the one the host waits for

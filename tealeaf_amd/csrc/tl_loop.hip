@@ -1,5 +1,6 @@
 // Device state, finishers and host side of the device-resident solver loops
 // (tl_loop.h).
+#include "tl_cg_pass.h"
 #include "tl_loop.h"
 #include "tealeaf_hip.h"
 
@@ -63,10 +64,10 @@ __global__ void __launch_bounds__(64) k_loop_base(State* st, int j0, int add)
 }
 
 // The stop rule and the report of iteration j (thread 0 of a finisher).
-__device__ void test_and_report(State* st, Slot* ring, int j, double rrn, const StopRule& rule)
+__device__ void test_and_report(State* st, Slot* ring, int j, double rrn, const StopRule& rule,
+                                int flags = 0)
 {
     const double err = rule.sqrt_err ? sqrt(rrn) : rrn;
-    int flags = 0;
     if (rule.rel ? rrn <= rule.rel_target : fabs(err) < rule.eps) flags |= kConverged;
     if (rule.sw == 1 && err < rule.eps_lim && j + 1 > 20) flags |= kSwitch;
     if (rule.sw == 2 && j + 1 > rule.presteps && err < 1.0) flags |= kSwitch;
@@ -111,6 +112,36 @@ k_loop_beta(unsigned nblocks, const double* __restrict__ partials, State* st, do
     blog[j] = b;
     st->rro = rrn;
     test_and_report(st, ring, j, rrn, rule);
+}
+
+__global__ void __launch_bounds__(64)
+k_loop_start(State* st, double rro, double alpha, double beta, double* alog, int j0)
+{
+    if (threadIdx.x == 0) {
+        st->rro = rro;
+        st->alpha = alpha;
+        st->beta = beta;
+        alog[j0] = alpha;
+    }
+}
+
+// The four sums of a CG pass (tl_cg_pass.h) end iteration j; the scalars
+// they give belong to the next one.
+__global__ void __launch_bounds__(256)
+k_loop_pass(unsigned nblocks, const double* __restrict__ partials, State* st, double* alog,
+            double* blog, int cap, Slot* ring, int j, int rel, StopRule rule)
+{
+    if (rel) j += st->base;
+    if (j > st->last) return;
+    double s[4];
+    tl_sum_partials<4>(nblocks, partials, s);
+    if (threadIdx.x != 0) return;
+    const double rrn = s[pass::kRR];
+    blog[j] = rrn / st->rro;
+    st->rro = rrn;
+    const bool fine = pass::scalars(s, &st->alpha, &st->beta);
+    if (j + 1 < cap) alog[j + 1] = st->alpha;
+    test_and_report(st, ring, j, rrn, rule, fine ? 0 : kCancel);
 }
 
 // The Jacobi error of iteration j: assigned (jacobi.c:99) or, for the
@@ -239,6 +270,30 @@ int finish_beta(unsigned nblocks, const StopRule& rule, const char* what)
     hipLaunchKernelGGL(k_loop_beta, dim3(1), dim3(256), 0, tl_stream(), nblocks,
                        tl_reduce_slots().partials, h.st, h.blog, h.ring, h.iter,
                        (int)h.capturing, rule);
+    return tl_check_launch(what);
+}
+
+int finish_pass(unsigned nblocks, const StopRule& rule, const char* what)
+{
+    Host& h = g_loop;
+    TL_TRY(check_finisher(nblocks, what));
+    if (!h.capturing) arm_slot(h.iter);
+    hipLaunchKernelGGL(k_loop_pass, dim3(1), dim3(256), 0, tl_stream(), nblocks,
+                       tl_reduce_slots().partials, h.st, h.alog, h.blog, h.cap, h.ring, h.iter,
+                       (int)h.capturing, rule);
+    return tl_check_launch(what);
+}
+
+int start_pass(int j0, const double sums[4])
+{
+    const char* what = "tl::loop::start_pass";
+    Host& h = g_loop;
+    if (!h.active || j0 < 0 || j0 >= h.cap)
+        return tl_fail(TLHIP_ERR_ARG, "%s: no resident loop is armed for iteration %d", what, j0);
+    double alpha, beta;
+    (void)pass::scalars(sums, &alpha, &beta);
+    hipLaunchKernelGGL(k_loop_start, dim3(1), dim3(64), 0, tl_stream(), h.st, sums[pass::kRR],
+                       alpha, beta, h.alog, j0);
     return tl_check_launch(what);
 }
 
