@@ -40,6 +40,21 @@ struct Outcome {
 int cg(const Plan& pl, double* u, double* p, double* r, const double* kx, const double* ky,
        const double* kz, int it0, int count, const loop::StopRule& rule, Outcome* out);
 
+// Chebyshev iterations it0, it0 + 1, ... with coefficients k0, k0 + 1, ...
+// (alphas[0], betas[0], ... on the host): at most `count`, fewer when the squared norm of r (its root with sqrt_err),
+// formed every tenth iteration from coefficient `est` on, falls below eps.
+// u, p and r in place (r is only written).  out->alpha: the last iteration
+// that formed the norm (rep), or -1.
+int cheby(const Plan& pl, double* u, double* p, double* r, const double* u0, const double* kx,
+          const double* ky, const double* kz, int it0, int count, int k0, int est,
+          const double* alphas, const double* betas, double eps, bool sqrt_err, Outcome* out);
+
+// Jacobi iterations it0, it0 + 1, ... of u in place; last_u: the interior
+// that the last one read.  rep: the last one's error.
+int jacobi(const Plan& pl, double* u, double* last_u, const double* u0, const double* kx,
+           const double* ky, const double* kz, int it0, int count, const loop::StopRule& rule,
+           Outcome* out);
+
 // Free the device and pinned memory (tlhip_finalise).
 void release();
 

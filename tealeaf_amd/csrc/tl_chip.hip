@@ -26,6 +26,12 @@
 // block also keeps r and p of its ring and updates them with that q, so the
 // ring's p equals the owner's bit for bit and no second meeting is needed.
 //
+// What bounds an iteration is the meeting: a block's sums reach the others in
+// about 1 us and are read back in another, beside 0.3 to 3 us of arithmetic
+// (1 to 8 cells per thread).  512^2 (K = 1) 4.4 us, 1024^2 (K = 4) 6.6, 128^3
+// (K = 8) 21; launch by launch they took 57, 76 and 63 us.  Chebyshev and
+// Jacobi, 1001 x 777: 4.9 us an iteration, 512^2: 4.4 us a sweep (25 and 13).
+//
 // Coherence: everything blocks exchange (q of outer cells, the sums) goes
 // through agent-scope atomic loads and stores, which the XCDs' L2s do not
 // hold back; a wave waits for its stores (vmcnt) before the block publishes
@@ -210,13 +216,22 @@ __device__ __forceinline__ bool all_sums(const double v[kSums], Shared& sh, doub
     return true;
 }
 
-__global__ void __launch_bounds__(256) k_empty(double* slots, int n)
+__global__ void __launch_bounds__(256) k_empty(double* slots, int n, unsigned* rounds)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < kMaxBlocks) rounds[i] = 0;
     if (i < n) slots[i] = __builtin_bit_cast(double, (unsigned long long)TL_MAIL_EMPTY);
 }
 
 // ------------------------------------------------------------ tile
+
+// An address part formed anew where it is used, so that the addresses of all
+// of a thread's cells are not kept in registers from iteration to iteration.
+__device__ __forceinline__ unsigned opaque(unsigned v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 // A thread's place in its tile, its cells' offsets in the fields and in LDS,
 // and its ring cells.
@@ -352,11 +367,7 @@ struct Tile {
     // Hand the tile's outer cells of v to the neighbours.
     __device__ __forceinline__ void hand_over(const double* v, double* xb) const
     {
-        // (an address is formed when it is used, not once for all iterations:
-        // 8 cells' addresses would take the registers of their fields)
-        unsigned at0 = xmine;
-        asm volatile("" : "+v"(at0));
-        double* my = xb + at0;
+        double* my = xb + opaque(xmine);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             const int m = DIMS == 2 ? t * K + k : k * RY + t;
@@ -416,12 +427,16 @@ struct Coefs {
         }
     }
 
-    // q = A s of the thread's cells, s in LDS with its ring, and s.q added to
-    // *dot; cells beyond a domain edge mirror the cell (a depth-1 reflective
-    // halo).  The association is 2d/shared.h:50-54 / 3d/shared.h:52-58.
-    // Cells outside the domain get 0.
-    __device__ __forceinline__ void apply(const T& tl, const double* s,
-                                          const double* s_k, double* dot, double q[K]) const
+    // f(k, c, x, y, z) for each of the thread's cells: the cell's value of s
+    // (in LDS with its ring) and per axis the two faces' coefficients and the
+    // values beyond them.  Cells beyond a domain edge mirror the cell (a
+    // depth-1 reflective halo).
+    struct Axis {
+        double kc, ku, lo, hi;        // lower and upper face, lower and upper neighbour
+    };
+    template <class F>
+    __device__ __forceinline__ void visit(const T& tl, const double* s, const double* s_k,
+                                          F&& f) const
     {
         const double* p = s + tl.at;
         double below = p[-tl.KP], c = p[0];
@@ -431,30 +446,179 @@ struct Coefs {
             double above = p[(k + 1) * tl.KP];
             const double next = above;
             if (tl.last_k && k == tl.kn - 1) above = c;
-            const double l = p[k * tl.KP + tl.lo], r = p[k * tl.KP + tl.hi];
             const double* sk = s_k + tl.k_at + k * tl.k_step;
-            double a;
+            const Axis along{kk[k], kk[k + 1], below, above};
+            Axis x{0.0, 0.0, p[k * tl.KP + tl.lo], p[k * tl.KP + tl.hi]};
             if constexpr (DIMS == 2) {
-                const double kxc = sk[0], kxr = sk[1];
-                const double d = (1.0 + (kxr + kxc)) + (kk[k + 1] + kk[k]);
-                a = d * c - (kxr * r + kxc * l) - (kk[k + 1] * above + kk[k] * below);
+                x.kc = sk[0];
+                x.ku = sk[1];
+                f(k, c, x, along, Axis{});
             } else {
-                const double kyc = sk[0], kyu = sk[tl.k_next], kxc = kx[k];
                 const double e = s_k[tl.e_at + k * tl.e_step];
-                double kxr = tl_lane_next(kxc, e);
-                if (tl.edge_x || tl.hi == 0) kxr = e;
-                const double so = p[k * tl.KP + tl.ylo], no = p[k * tl.KP + tl.yhi];
-                const double d = ((1.0 + (kxr + kxc)) + (kyu + kyc)) + (kk[k + 1] + kk[k]);
-                a = d * c - (kxr * r + kxc * l) - (kyu * no + kyc * so)
-                    - (kk[k + 1] * above + kk[k] * below);
+                x.kc = kx[k];
+                x.ku = tl_lane_next(x.kc, e);
+                if (tl.edge_x || tl.hi == 0) x.ku = e;
+                const Axis y{sk[0], sk[tl.k_next], p[k * tl.KP + tl.ylo], p[k * tl.KP + tl.yhi]};
+                f(k, c, x, y, along);
             }
-            q[k] = k < tl.kn ? a : 0.0;
-            *dot += q[k] * c;
             below = c;
             c = next;
         }
     }
+
+    // A s at a cell; the association is 2d/shared.h:50-54 / 3d/shared.h:52-58.
+    static __device__ __forceinline__ double product(double c, const Axis& x, const Axis& y,
+                                                     const Axis& z)
+    {
+        const double d = (1.0 + (x.ku + x.kc)) + (y.ku + y.kc);
+        const double a = (DIMS == 2 ? d : d + (z.ku + z.kc)) * c - (x.ku * x.hi + x.kc * x.lo)
+                         - (y.ku * y.hi + y.kc * y.lo);
+        return DIMS == 2 ? a : a - (z.ku * z.hi + z.kc * z.lo);
+    }
+
+    // q = A s of the thread's cells (0 outside the domain), and s.q added to
+    // *dot.
+    __device__ __forceinline__ void apply(const T& tl, const double* s, const double* s_k,
+                                          double* dot, double q[K]) const
+    {
+        visit(tl, s, s_k, [&](int k, double c, const Axis& x, const Axis& y, const Axis& z) {
+            q[k] = k < tl.kn ? product(c, x, y, z) : 0.0;
+            *dot += q[k] * c;
+        });
+    }
 };
+
+// The ring of a field in LDS: where each of the block's ring cells is and
+// where its owner hands it over.
+template <int DIMS, int K, int LXS>
+struct Ring {
+    using T = Tile<DIMS, K, LXS>;
+    static constexpr int NE = T::NE;
+    int dst[NE];            // < 0: none
+    unsigned src[NE];
+    bool zl, zh;            // 3D: the cells below and above this thread's
+
+    // load(slot, LDS index, cell) for every ring cell there is; slots NE and
+    // NE + 1 are the z cells (a tile with a neighbour above is full along z)
+    template <class F>
+    __device__ __forceinline__ void init(const Geo& g, const T& tl, F&& load)
+    {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            unsigned from = 0;
+            long cell = 0;
+            bool in = false;
+            int to = 0;
+            dst[i] = -1;
+            src[i] = 0;
+            if (tl.ring(g, (int)threadIdx.x + i * kThreads, &to, &from, &cell, &in) && in) {
+                dst[i] = to;
+                src[i] = from;
+                load(i, to, cell);
+            }
+        }
+        zl = DIMS == 3 && tl.face_zl && tl.kn > 0;
+        zh = DIMS == 3 && tl.face_zh && tl.kn > 0;
+        if (zl) load(NE, tl.at - tl.KP, (long)tl.first - tl.kstep);
+        if (zh) load(NE + 1, tl.at + K * tl.KP, (long)tl.first + (long)K * tl.kstep);
+    }
+
+    // What the owners handed over, on its way; use() gives it to
+    // put(slot, LDS index, value).  Between the two there is time for work
+    // that does not need it.
+    struct Handed {
+        double v[NE], w[2];
+    };
+    __device__ __forceinline__ Handed fetch(const Geo& g, const T& tl, const double* xb) const
+    {
+        Handed h;
+#pragma unroll
+        for (int i = 0; i < NE; ++i) h.v[i] = dst[i] >= 0 ? ld_agent(&xb[src[i]]) : 0.0;
+        h.w[0] = zl ? ld_agent(&xb[tl.zlow(g)]) : 0.0;
+        h.w[1] = zh ? ld_agent(&xb[tl.zhigh(g)]) : 0.0;
+        return h;
+    }
+    template <class F>
+    __device__ __forceinline__ void use(const T& tl, const Handed& h, F&& put) const
+    {
+#pragma unroll
+        for (int i = 0; i < NE; ++i)
+            if (dst[i] >= 0) put(i, dst[i], h.v[i]);
+        if (zl) put(NE, tl.at - tl.KP, h.w[0]);
+        if (zh) put(NE + 1, tl.at + K * tl.KP, h.w[1]);
+    }
+};
+
+// Wait until the blocks this one shares a face with have handed over their
+// cells of round n (1, 2, ...).  What is handed over alternates between two
+// buffers: a block writes a buffer again two rounds later, after its
+// neighbours have published the round between, which they do after they read
+// it.
+template <class T>
+__device__ __forceinline__ bool meet_neighbours(const Geo& g, const T& tl, unsigned* rounds,
+                                                unsigned n, Shared& sh)
+{
+    const int tid = threadIdx.x, b = blockIdx.x;
+    wait_stores();
+    __syncthreads();
+    if (tid == 0) __hip_atomic_store(&rounds[b], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid < 6) {
+        const int step[3] = {1, g.tx, g.tx * g.ty};
+        const bool have[6] = {tl.face_xl, tl.face_xh, tl.face_yl, tl.face_yh, tl.face_zl, tl.face_zh};
+        bool mine = false;
+        int at = b;
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+            if (tid == i) {
+                mine = have[i];
+                at = b + (i & 1 ? step[i >> 1] : -step[i >> 1]);
+            }
+        if (mine) {
+            unsigned spin = 0;
+            unsigned long long t0 = 0;
+            while (__hip_atomic_load(&rounds[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n) {
+                if ((++spin & 255u) == 0) {
+                    const unsigned long long now = __builtin_amdgcn_s_memrealtime();   // 100 MHz
+                    if (!t0) t0 = now;
+                    if (now - t0 > (unsigned long long)(kWaitS * 1e8)) {
+                        sh.expired = 1;
+                        break;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    return !sh.expired;
+}
+
+// A kernel's start: p's place in LDS zeroed (outside the domain and in a
+// ring without neighbours, where the mirror is read instead, it stays zero),
+// the coefficients loaded.
+template <int DIMS, int K, int LXS>
+__device__ __forceinline__ void begin_tile(const Geo& g, const Tile<DIMS, K, LXS>& tl,
+                                           Coefs<DIMS, K, LXS>& co, double* s, double* s_k,
+                                           Shared& sh, const double* kx, const double* ky,
+                                           const double* kz)
+{
+    if (threadIdx.x == 0) sh.expired = 0;
+    for (int i = threadIdx.x; i < lds_p<DIMS, K>(LXS); i += kThreads) s[i] = 0.0;
+    for (int i = threadIdx.x; i < lds_k<DIMS, K>(LXS); i += kThreads) s_k[i] = 0.0;
+    __syncthreads();
+    co.load(g, tl, s_k, kx, ky, kz);
+}
+
+// The run's outcome to the host, by one thread of the grid.
+__device__ __forceinline__ void report(Mail* mail, double rrn, double err, int flags, int last,
+                                       double a, double b)
+{
+    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    const double m[6] = {rrn, err, (double)flags, (double)last, a, b};
+    double* to = &mail->rrn;
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+        __hip_atomic_store(to + i, m[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // ------------------------------------------------------------ CG
 
@@ -487,16 +651,9 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
     double* s_p = lds;
     double* s_k = lds + lds_p<DIMS, K>(LXS);
     const int nb = (int)gridDim.x;
-    if (threadIdx.x == 0) sh.expired = 0;
     constexpr int NE = decltype(tl)::NE;
-
-    // p is zero outside the domain and in a ring without neighbours, where
-    // the mirror is read instead
-    for (int i = threadIdx.x; i < lds_p<DIMS, K>(LXS); i += kThreads) s_p[i] = 0.0;
-    for (int i = threadIdx.x; i < lds_k<DIMS, K>(LXS); i += kThreads) s_k[i] = 0.0;
-    __syncthreads();
     Coefs<DIMS, K, LXS> co;
-    co.load(g, tl, s_k, A.kx, A.ky, A.kz);
+    begin_tile(g, tl, co, s_p, s_k, sh, A.kx, A.ky, A.kz);
     double r[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -506,38 +663,15 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
         if (in) s_p[tl.at + k * tl.KP] = A.p[c];
     }
     // the ring: r in registers, p in LDS
-    double rr[NE], rz[2] = {0.0, 0.0};
-    int rdst[NE];
-    unsigned rsrc[NE];
-#pragma unroll
-    for (int i = 0; i < NE; ++i) {
-        unsigned src = 0;
-        long cell = 0;
-        bool in = false;
-        int dst = 0;
-        rr[i] = 0.0;
-        rdst[i] = -1;
-        rsrc[i] = 0;
-        if (tl.ring(g, (int)threadIdx.x + i * kThreads, &dst, &src, &cell, &in) && in) {
-            rr[i] = A.r[cell];
-            s_p[dst] = A.p[cell];
-            rdst[i] = dst;
-            rsrc[i] = src;
-        }
-    }
-    // the cells below and above this thread's (a tile with a neighbour above
-    // is full along z)
-    const bool zl = DIMS == 3 && tl.face_zl && tl.kn > 0, zh = DIMS == 3 && tl.face_zh && tl.kn > 0;
-    if (zl) {
-        rz[0] = A.r[tl.first - tl.kstep];
-        s_p[tl.at - tl.KP] = A.p[tl.first - tl.kstep];
-    }
-    if (zh) {
-        rz[1] = A.r[tl.first + K * tl.kstep];
-        s_p[tl.at + K * tl.KP] = A.p[tl.first + K * tl.kstep];
-    }
+    double rr[NE + 2] = {};
+    Ring<DIMS, K, LXS> ring;
+    ring.init(g, tl, [&](int i, int to, long cell) {
+        rr[i] = A.r[cell];
+        s_p[to] = A.p[cell];
+    });
     __syncthreads();
 
+    const unsigned any_cell = (unsigned)(g.hd + (long)g.hd * g.x + (DIMS == 3 ? g.hd * g.xy : 0));
     double prev = 0.0, alpha = 0.0, beta_true = 0.0;
     double rrn = 0.0, err = 0.0;
     int flags = 0, n = 0, meeting = 0;
@@ -557,9 +691,10 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
         constexpr bool kEarlyU = K <= 2;
         double u[kEarlyU ? K : 1];
         if constexpr (kEarlyU) {
+            // (every lane loads something: a load that only some paths wait
+            // for makes the next iteration wait for this one's stores)
 #pragma unroll
-            for (int k = 0; k < K; ++k)
-                u[k] = go_on && k < tl.kn ? A.u[tl.first + k * tl.kstep] : 0.0;
+            for (int k = 0; k < K; ++k) u[k] = A.u[k < tl.kn ? tl.first + k * tl.kstep : any_cell];
         }
         if (!all_sums(v, sh, A.slots, meeting++, nb, tot)) {
             flags = -1;
@@ -580,26 +715,21 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
         const double predicted = (rro - 2.0 * alpha * tot[2]) + alpha * alpha * tot[1];
         double beta = predicted / rro;
         if (blockIdx.x == 0 && threadIdx.x == 0) A.alog[A.it0 + n] = alpha;
-        double qr[NE], qz[2] = {0.0, 0.0};
-        if (nb > 1) {
-#pragma unroll
-            for (int i = 0; i < NE; ++i) qr[i] = rdst[i] >= 0 ? ld_agent(&xb[rsrc[i]]) : 0.0;
-            if (zl) qz[0] = ld_agent(&xb[tl.zlow(g)]);
-            if (zh) qz[1] = ld_agent(&xb[tl.zhigh(g)]);
-        }
-        unsigned cell0 = tl.first;
-        asm volatile("" : "+v"(cell0));
+        typename decltype(ring)::Handed handed{};
+        if (nb > 1) handed = ring.fetch(g, tl, xb);
+        const unsigned cell0 = opaque(tl.first);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            if (k < tl.kn) {
-                double* ug = A.u + cell0 + k * tl.kstep;
-                double uk;
-                if constexpr (kEarlyU) uk = u[k];
-                else uk = *ug;
-                uk += alpha * s_p[tl.at + k * tl.KP];
-                r[k] -= alpha * q[k];
-                *ug = uk;
+            // outside the domain p, q and r are zero, and stay so
+            const double step = alpha * s_p[tl.at + k * tl.KP];
+            double* ug = A.u + cell0 + k * tl.kstep;
+            if constexpr (kEarlyU) {
+                u[k] += step;
+                if (k < tl.kn) *ug = u[k];
+            } else if (k < tl.kn) {
+                *ug += step;
             }
+            r[k] -= alpha * q[k];
             if (K == 8 && k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
         if (!(predicted >= 0.01 * rro)) {          // the same decision in every block
@@ -616,21 +746,10 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
         for (int k = 0; k < K; ++k)
             if (k < tl.kn) s_p[tl.at + k * tl.KP] = beta * s_p[tl.at + k * tl.KP] + r[k];
         if (nb > 1) {
-#pragma unroll
-            for (int i = 0; i < NE; ++i) {
-                if (rdst[i] >= 0) {
-                    rr[i] -= alpha * qr[i];
-                    s_p[rdst[i]] = beta * s_p[rdst[i]] + rr[i];
-                }
-            }
-            if (zl) {
-                rz[0] -= alpha * qz[0];
-                s_p[tl.at - tl.KP] = beta * s_p[tl.at - tl.KP] + rz[0];
-            }
-            if (zh) {
-                rz[1] -= alpha * qz[1];
-                s_p[tl.at + K * tl.KP] = beta * s_p[tl.at + K * tl.KP] + rz[1];
-            }
+            ring.use(tl, handed, [&](int i, int at, double q_ring) {
+                rr[i] -= alpha * q_ring;
+                s_p[at] = beta * s_p[at] + rr[i];
+            });
         }
         __syncthreads();
     }
@@ -643,13 +762,227 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
             A.p[c] = s_p[tl.at + k * tl.KP];
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const double m[6] = {rrn, err, (double)flags, (double)(A.it0 + n - 1), alpha, beta_true};
-        double* to = &A.mail->rrn;
+    report(A.mail, rrn, err, flags, A.it0 + n - 1, alpha, beta_true);
+}
+
+// ------------------------------------------------------------ Chebyshev
+
+// A field that the loop only reads at a thread's own cells: in registers, or
+// with 8 cells per thread, which leave none, from the L2 each time.
+template <int DIMS, int K, int LXS>
+struct Steady {
+    static constexpr bool kHeld = K < 8;
+    double v[kHeld ? K : 1];
+    const double* f;
+    unsigned step;
+    int kn;
+    __device__ __forceinline__ Steady(const Tile<DIMS, K, LXS>& tl, const double* field)
+        : f(field), step(tl.kstep), kn(tl.kn)
+    {
+        if constexpr (kHeld)
 #pragma unroll
-        for (int i = 0; i < 6; ++i)
-            __hip_atomic_store(to + i, m[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            for (int k = 0; k < K; ++k)
+                v[k] = k < kn ? f[tl.first + k * step] : 0.0;
     }
+    __device__ __forceinline__ double operator()(int k, unsigned cell0) const
+    {
+        if constexpr (kHeld) return v[k];
+        else return k < kn ? f[cell0 + k * step] : 0.0;
+    }
+};
+
+struct ChebyArgs {
+    Geo g;
+    double *u, *p, *r;
+    const double *u0, *kx, *ky, *kz;
+    double *xbuf, *slots;
+    unsigned* rounds;
+    Mail* mail;
+    const double *alphas, *betas;     // of the run's iterations
+    int it0, count, k0, est;
+    double eps;
+    int sqrt_err;
+};
+
+// Iterations of the Chebyshev loop (2d/drivers/cheby_driver.c with
+// cheby.c:57-85): w = A u, r = u0 - w, p = alpha p + beta r, u += p.  Blocks
+// meet their neighbours only, except where the norm of r is due (every tenth
+// iteration from the estimate on).
+template <int DIMS, int K, int LXS>
+__global__ void __launch_bounds__(kThreads) k_chip_cheby(ChebyArgs A)
+{
+    extern __shared__ double lds[];
+    __shared__ Shared sh;
+    const Geo& g = A.g;
+    const Tile<DIMS, K, LXS> tl(g);
+    double* s_u = lds;
+    double* s_k = lds + lds_p<DIMS, K>(LXS);
+    const int nb = (int)gridDim.x;
+    Coefs<DIMS, K, LXS> co;
+    begin_tile(g, tl, co, s_u, s_k, sh, A.kx, A.ky, A.kz);
+    double p[K];
+    const Steady<DIMS, K, LXS> u0(tl, A.u0);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const bool in = k < tl.kn;
+        const long c = tl.first + k * tl.kstep;
+        p[k] = in ? A.p[c] : 0.0;
+        if (in) s_u[tl.at + k * tl.KP] = A.u[c];
+    }
+    Ring<DIMS, K, LXS> ring;
+    ring.init(g, tl, [&](int, int to, long cell) { s_u[to] = A.u[cell]; });
+    __syncthreads();
+
+    double rrn = 0.0, err = 0.0, normed = -1.0;
+    int flags = 0, n = 0, meeting = 0;
+    for (;; ++n) {
+        const double alpha = A.alphas[n], beta = A.betas[n];
+        double un[K], v[kSums] = {0.0, 0.0, 0.0, 0.0};
+        const int t = A.it0 + n;
+        const bool norm = A.k0 + n >= A.est && (t + 1) % 10 == 0;
+        const bool keep_r = norm || n + 1 >= A.count;        // it may end here
+        const unsigned cell0 = opaque(tl.first);
+        co.visit(tl, s_u, s_k, [&](int k, double c, const auto& x, const auto& y, const auto& z) {
+            const double r = u0(k, cell0) - co.product(c, x, y, z);
+            p[k] = alpha * p[k] + beta * r;
+            un[k] = c + p[k];
+            if (k < tl.kn) {
+                v[0] += r * r;
+                if (keep_r) A.r[cell0 + k * tl.kstep] = r;
+            }
+        });
+        __syncthreads();          // everybody has read the old u
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (k < tl.kn) s_u[tl.at + k * tl.KP] = un[k];
+        double* xb = A.xbuf + (size_t)(n & 1) * tl.xall;
+        if (nb > 1) tl.hand_over(un, xb);
+        bool fine = true;
+        if (norm) {
+            double tot[kSums];
+            fine = all_sums(v, sh, A.slots, meeting++, nb, tot);
+            rrn = tot[0];
+            err = A.sqrt_err ? sqrt(rrn) : rrn;
+            normed = t;
+            if (fabs(err) < A.eps) flags = loop::kConverged;
+        } else if (nb > 1) {
+            fine = meet_neighbours(g, tl, A.rounds, n + 1, sh);
+        }
+        if (!fine) {
+            flags = -1;
+            break;
+        }
+        if (flags || n + 1 >= A.count) break;
+        if (nb > 1) {
+            ring.use(tl, ring.fetch(g, tl, xb), [&](int, int to, double v) { s_u[to] = v; });
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (k < tl.kn) {
+            const long c = tl.first + k * tl.kstep;
+            A.u[c] = s_u[tl.at + k * tl.KP];
+            A.p[c] = p[k];
+        }
+    }
+    report(A.mail, rrn, err, flags, A.it0 + n, normed, 0.0);
+}
+
+// ------------------------------------------------------------ Jacobi
+
+struct JacobiArgs {
+    Geo g;
+    double *u, *last_u;
+    const double *u0, *kx, *ky, *kz;
+    double *xbuf, *slots;
+    Mail* mail;
+    int it0, count;
+    loop::StopRule rule;
+};
+
+// Jacobi sweeps (jacobi.c:61-100): the error, the sum of |change|, is due
+// every iteration, so the blocks all meet; every 50th iteration the squared
+// norm of the residual is added to it (jacobi_driver.c:22-40).
+template <int DIMS, int K, int LXS>
+__global__ void __launch_bounds__(kThreads) k_chip_jacobi(JacobiArgs A)
+{
+    extern __shared__ double lds[];
+    __shared__ Shared sh;
+    const Geo& g = A.g;
+    const Tile<DIMS, K, LXS> tl(g);
+    double* s_u = lds;
+    double* s_k = lds + lds_p<DIMS, K>(LXS);
+    const int nb = (int)gridDim.x;
+    Coefs<DIMS, K, LXS> co;
+    begin_tile(g, tl, co, s_u, s_k, sh, A.kx, A.ky, A.kz);
+    double old[K];
+    const Steady<DIMS, K, LXS> u0(tl, A.u0);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (k < tl.kn) s_u[tl.at + k * tl.KP] = A.u[tl.first + k * tl.kstep];
+    Ring<DIMS, K, LXS> ring;
+    ring.init(g, tl, [&](int, int to, long cell) { s_u[to] = A.u[cell]; });
+    __syncthreads();
+
+    double e = 0.0, err = 0.0;
+    int flags = 0, n = 0, meeting = 0;
+    for (;; ++n) {
+        double un[K], v[kSums] = {0.0, 0.0, 0.0, 0.0}, tot[kSums];
+        const unsigned cell0 = opaque(tl.first);
+        co.visit(tl, s_u, s_k, [&](int k, double c, const auto& x, const auto& y, const auto& z) {
+            double num = (u0(k, cell0) + (x.ku * x.hi + x.kc * x.lo)) + (y.ku * y.hi + y.kc * y.lo);
+            double den = (1.0 + (x.kc + x.ku)) + (y.kc + y.ku);
+            if constexpr (DIMS == 3) {
+                num = num + (z.ku * z.hi + z.kc * z.lo);
+                den = den + (z.kc + z.ku);
+            }
+            un[k] = num / den;
+            old[k] = c;
+            if (k < tl.kn) v[0] += fabs(un[k] - c);
+        });
+        __syncthreads();          // everybody has read the old u
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (k < tl.kn) s_u[tl.at + k * tl.KP] = un[k];
+        double* xb = A.xbuf + (size_t)(n & 1) * tl.xall;
+        if (nb > 1) tl.hand_over(un, xb);
+        if (!all_sums(v, sh, A.slots, meeting++, nb, tot)) {
+            flags = -1;
+            break;
+        }
+        if (nb > 1) {
+            ring.use(tl, ring.fetch(g, tl, xb), [&](int, int to, double w) { s_u[to] = w; });
+        }
+        __syncthreads();
+        e = tot[0];
+        const int t = A.it0 + n;
+        if (t % 50 == 0) {
+            double w[kSums] = {0.0, 0.0, 0.0, 0.0};
+            co.visit(tl, s_u, s_k,
+                     [&](int k, double c, const auto& x, const auto& y, const auto& z) {
+                         const double d = u0(k, cell0) - co.product(c, x, y, z);
+                         if (k < tl.kn) w[0] += d * d;
+                     });
+            if (!all_sums(w, sh, A.slots, meeting++, nb, tot)) {
+                flags = -1;
+                break;
+            }
+            e = e + tot[0];
+        }
+        err = A.rule.sqrt_err ? sqrt(e) : e;
+        flags = stop_flags(A.rule, t, e, err);
+        if (flags || n + 1 >= A.count) break;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (k < tl.kn) {
+            const long c = tl.first + k * tl.kstep;
+            A.u[c] = s_u[tl.at + k * tl.KP];
+            A.last_u[c] = old[k];
+        }
+    }
+    report(A.mail, e, err, flags, A.it0 + n, 0.0, 0.0);
 }
 
 // ------------------------------------------------------------ host
@@ -658,6 +991,8 @@ struct Host {
     double* xbuf = nullptr;
     size_t xlen = 0;
     double* slots = nullptr;
+    unsigned* rounds = nullptr;
+    double* coefs = nullptr;      // [2 * kChunk]
     Mail* mail = nullptr;
     int cus = 0;
 };
@@ -722,6 +1057,7 @@ int prepare(int nb, size_t xdoubles, const char* what)
     TL_TRY(tl_ensure_init());
     if (!h.slots) {
         CHIP_HIP(hipMalloc(&h.slots, sizeof(double) * kPhases * kMaxBlocks * kSums), what);
+        CHIP_HIP(hipMalloc(&h.rounds, sizeof(unsigned) * kMaxBlocks), what);
         CHIP_HIP(hipHostMalloc(&h.mail, sizeof(Mail), hipHostMallocMapped | hipHostMallocCoherent),
                  what);
     }
@@ -735,7 +1071,7 @@ int prepare(int nb, size_t xdoubles, const char* what)
     }
     if (nb == 1) return 0;        // a single block has nobody to meet
     const int n = kPhases * kMaxBlocks * kSums;
-    hipLaunchKernelGGL(k_empty, dim3((n + 255) / 256), dim3(256), 0, tl_stream(), h.slots, n);
+    hipLaunchKernelGGL(k_empty, dim3((n + 255) / 256), dim3(256), 0, tl_stream(), h.slots, n, h.rounds);
     return tl_check_launch(what);
 }
 
@@ -813,8 +1149,11 @@ Plan plan(int dims, int x, int y, int z, int hd)
     const int nx = x - 2 * hd, ny = y - 2 * hd, nz = dims == 3 ? z - 2 * hd : 1;
     if (nx < 1 || ny < 1 || nz < 1) return best;
     const int most = std::min(kMaxBlocks, compute_units());
-    // One meeting costs what about eight more cells per thread do, so a grid
-    // that fits one block runs in one; otherwise the fewest cells per thread.
+    // A block per CU at most: blocks wait for each other.  The fewest cells
+    // per thread that fit are fastest (us per CG iteration with 1, 2, 4, 8
+    // cells: 512^2 5.6 5.5 6.1 8.5; 1024^2 - - 7.3 9.7; 64^3 - 8.5 9.4 17.2),
+    // except that a grid which fits one block needs no meeting across the
+    // chip (48^2, one block 3.7 us a sweep, several 4.3).
     double cost = 1e30;
     for (int k = 1; k <= 8; k *= 2) {
         for (int lxs = 6; lxs >= 4; --lxs) {
@@ -836,40 +1175,109 @@ Plan plan(int dims, int x, int y, int z, int hd)
     return best;
 }
 
-int cg(const Plan& pl, double* u, double* p, double* r, const double* kx, const double* ky,
-       const double* kz, int it0, int count, const loop::StopRule& rule, Outcome* out)
+namespace {
+// Launch one of the loops, args(g) giving its arguments, and wait for its
+// report.
+template <template <int, int, int> class Kernel, class Args>
+int run(const Plan& pl, int count, const char* what, Args&& args, Mail* m)
 {
-    const char* what = "tl::chip::cg";
     if (!pl.ok) return tl_fail(TLHIP_ERR_ARG, "%s: the grid does not fit", what);
     if (count < 1) return tl_fail(TLHIP_ERR_ARG, "%s: no iteration to run", what);
     return with_plan(pl, [&](auto dims, auto kc, auto row) -> int {
         constexpr int D = decltype(dims)::value, K = decltype(kc)::value;
         constexpr int LXS = decltype(row)::value;
-        const Geo g = geo_of(pl);
         const int nb = pl.blocks();
-        TL_TRY(prepare(nb, 2 * (size_t)nb * faces_of<D, K>(pl.lxs).total(), what));
-        const size_t lds = lds_bytes<D, K>(pl.lxs);
-        const void* fn = (const void*)k_chip_cg<D, K, LXS>;
+        TL_TRY(prepare(nb, 2 * (size_t)nb * faces_of<D, K>(LXS).total(), what));
+        const size_t lds = lds_bytes<D, K>(LXS);
+        const void* fn = Kernel<D, K, LXS>::fn();
         CHIP_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), what);
-        CgArgs a{g, u, p, r, kx, ky, kz, g_chip.xbuf, g_chip.slots, nullptr, nullptr, g_chip.mail,
-                 it0, (int)std::min<long>(count, kChunk), rule};
-        loop::log_ptrs(&a.alog, &a.blog);
+        auto a = args(geo_of(pl));
         arm_mail();
-        void* args[] = {&a};
-        CHIP_HIP(hipLaunchCooperativeKernel(fn, dim3(nb), dim3(kThreads), args, (unsigned)lds,
+        void* ptrs[] = {&a};
+        const int slot = tl_timer_begin(what);
+        CHIP_HIP(hipLaunchCooperativeKernel(fn, dim3(nb), dim3(kThreads), ptrs, (unsigned)lds,
                                             tl_stream()), what);
-        Mail m;
-        TL_TRY(wait_mail(&m, what));
-        if (m.flags < 0.0)
+        tl_timer_end(slot);
+        TL_TRY(wait_mail(m, what));
+        if (m->flags < 0.0)
             return tl_fail(TLHIP_ERR_HIP, "%s: a block waited over %.0f s for another", what, kWaitS);
-        out->rep.rrn = m.rrn;
-        out->rep.err = m.err;
-        out->rep.flags = (int)m.flags;
-        out->last = (int)m.last;
-        out->alpha = m.alpha;
-        out->beta = m.beta;
         return 0;
     });
+}
+
+template <int D, int K, int L> struct Cg {
+    static const void* fn() { return (const void*)k_chip_cg<D, K, L>; }
+};
+template <int D, int K, int L> struct Cheby {
+    static const void* fn() { return (const void*)k_chip_cheby<D, K, L>; }
+};
+template <int D, int K, int L> struct Jacobi {
+    static const void* fn() { return (const void*)k_chip_jacobi<D, K, L>; }
+};
+
+void outcome(const Mail& m, Outcome* out)
+{
+    out->rep.rrn = m.rrn;
+    out->rep.err = m.err;
+    out->rep.flags = (int)m.flags;
+    out->last = (int)m.last;
+    out->alpha = m.alpha;
+    out->beta = m.beta;
+}
+}  // namespace
+
+int cg(const Plan& pl, double* u, double* p, double* r, const double* kx, const double* ky,
+       const double* kz, int it0, int count, const loop::StopRule& rule, Outcome* out)
+{
+    Mail m;
+    double *alog, *blog;
+    loop::log_ptrs(&alog, &blog);
+    const int cnt = (int)std::min<long>(count, kChunk);
+    TL_TRY((run<Cg>(pl, cnt, "tl_chip_cg", [&](const Geo& g) {
+        return CgArgs{g, u, p, r, kx, ky, kz, g_chip.xbuf, g_chip.slots, alog, blog, g_chip.mail,
+                      it0, cnt, rule};
+    }, &m)));
+    outcome(m, out);
+    return 0;
+}
+
+int cheby(const Plan& pl, double* u, double* p, double* r, const double* u0, const double* kx,
+          const double* ky, const double* kz, int it0, int count, int k0, int est,
+          const double* alphas, const double* betas, double eps, bool sqrt_err, Outcome* out)
+{
+    const char* what = "tl_chip_cheby";
+    Mail m;
+    const int cnt = (int)std::min<long>(count, kChunk);
+    TL_TRY(tl_ensure_init());
+    Host& h = g_chip;
+    if (!h.coefs) CHIP_HIP(hipMalloc(&h.coefs, sizeof(double) * 2 * kChunk), what);
+    if (cnt > 0) {
+        const size_t bytes = sizeof(double) * cnt;
+        CHIP_HIP(hipMemcpyAsync(h.coefs, alphas, bytes, hipMemcpyHostToDevice, tl_stream()), what);
+        CHIP_HIP(hipMemcpyAsync(h.coefs + kChunk, betas, bytes, hipMemcpyHostToDevice, tl_stream()),
+                 what);
+    }
+    TL_TRY((run<Cheby>(pl, cnt, what, [&](const Geo& g) {
+        return ChebyArgs{g, u, p, r, u0, kx, ky, kz, g_chip.xbuf, g_chip.slots, g_chip.rounds,
+                         g_chip.mail, g_chip.coefs, g_chip.coefs + kChunk, it0, cnt, k0, est, eps,
+                         (int)sqrt_err};
+    }, &m)));
+    outcome(m, out);
+    return 0;
+}
+
+int jacobi(const Plan& pl, double* u, double* last_u, const double* u0, const double* kx,
+           const double* ky, const double* kz, int it0, int count, const loop::StopRule& rule,
+           Outcome* out)
+{
+    Mail m;
+    const int cnt = (int)std::min<long>(count, kChunk);
+    TL_TRY((run<Jacobi>(pl, cnt, "tl_chip_jacobi", [&](const Geo& g) {
+        return JacobiArgs{g, u, last_u, u0, kx, ky, kz, g_chip.xbuf, g_chip.slots, g_chip.mail, it0,
+                          cnt, rule};
+    }, &m)));
+    outcome(m, out);
+    return 0;
 }
 
 void release()
@@ -877,6 +1285,8 @@ void release()
     Host& h = g_chip;
     if (h.xbuf) (void)hipFree(h.xbuf);
     if (h.slots) (void)hipFree(h.slots);
+    if (h.rounds) (void)hipFree(h.rounds);
+    if (h.coefs) (void)hipFree(h.coefs);
     if (h.mail) (void)hipHostFree(h.mail);
     h = Host{};
 }

@@ -1057,6 +1057,24 @@ struct tlhip_problem {
                 TRY(halo_update(1));
                 TRY(cheby_step(ncheby, true, error));
                 est = est_iterations(*error, bb);
+            } else if (chip_cheby()) {
+                // all the iterations up to the stop in one launch (one per
+                // launch without fusion)
+                const int from = tt;
+                tl::chip::Outcome o;
+                TRY(tl::chip::cheby(chip, u, p, r, u0, kx, ky, kz, tt,
+                                    g_cheby_fusion > 1 ? s.max_iters - tt : 1, ncheby, est,
+                                    &cheby_alphas[ncheby], &cheby_betas[ncheby], s.eps, dims == 3,
+                                    &o));
+                rep->n_cheby_steps += o.last - from + 1;
+                ncheby += o.last - from;
+                tt = o.last;
+                const int normed = (int)o.alpha;
+                if (normed >= 0) *error = o.rep.rrn;
+                // 3D takes the root of the error at every iteration's test,
+                // whether that iteration formed it or not
+                if (dims == 3)
+                    for (int j = normed >= 0 ? normed : from; j < tt; ++j) *error = std::sqrt(*error);
             } else if (fused_cheby()) {
                 // Iterations tt, tt+1, ... in one pass, up to and including
                 // the next one that computes the norm (the only ones after
@@ -1094,6 +1112,13 @@ struct tlhip_problem {
         rep->printed_inner_iters = ncheby;
         rep->est_iters = est;
         return 0;
+    }
+
+    // Chebyshev iterations of grids that fit the chip, many to a launch
+    // (tl_chip.h); the reference's own stop test, as fused_cheby.
+    bool chip_cheby() const
+    {
+        return chip.ok && interior() && rel_tol <= 0.0 && (dims == 2 || s.eps < 1.0);
     }
 
     // Several Chebyshev iterations per pass (2D).  With the relative stop
@@ -1534,6 +1559,20 @@ struct tlhip_problem {
         if (g_resident && interior()) return jacobi_resident(error);
         int tt;
         for (tt = 0; tt < s.max_iters; ++tt) {
+            if (chip_jacobi()) {
+                // one iteration of the resident loop's launch: the same bits
+                tl::loop::StopRule never{};
+                never.eps = -1.0;
+                int last;
+                tl::loop::Report rp;
+                TRY(jacobi_chip(tt, 1, never, &last, &rp));
+                rep->n_jacobi++;
+                *error = rp.rrn;
+                bool done;
+                TRY(stop(error, &done));
+                if (done) break;
+                continue;
+            }
             if (dims == 2) TRY(tlhip2d_jacobi_iterate(x, y, hd, error, kx, ky, u0, u, r));
             else TRY(tlhip3d_jacobi_solver_iterate(x, y, z, hd, error, kx, ky, kz, u0, u, r));
             rep->n_jacobi++;
@@ -1557,8 +1596,53 @@ struct tlhip_problem {
     // the same and u ends as the host-driven loop leaves it.  r is then made
     // what the host-driven loop leaves: the last sweep's input, with the
     // residual in its interior when that iteration computed one.
+    // Jacobi iterations of grids that fit the chip, many to a launch.  Not in
+    // 3D with 8 cells per thread: the sweep's division leaves too few
+    // registers (128^3: 46 us a sweep against 24 us with the sweep's own
+    // launches; 80^3, 4 cells per thread: 6.9 against 14 us).
+    bool chip_jacobi() const { return chip.ok && interior() && !(dims == 3 && chip.k == 8); }
+
+    // At most count iterations from t0 in one launch (tl_chip.h).  r then
+    // holds what the loop leaves there: the last sweep's input, halo included
+    // (before the first sweep that is u's as it stands), with the residual
+    // in its interior when that iteration computed one.
+    int jacobi_chip(int t0, int count, const tl::loop::StopRule& rule, int* last,
+                    tl::loop::Report* rp)
+    {
+        TRY(tlhip_copy_device(r, u, sizeof(double) * (size_t)n));
+        tl::chip::Outcome o;
+        TRY(tl::chip::jacobi(chip, u, r, u0, kx, ky, kz, t0, count, rule, &o));
+        if (o.last > t0) {
+            std::swap(u, r);
+            const int rc = halo_update(1);
+            std::swap(u, r);
+            TRY(rc);
+        }
+        TRY(halo_update(1));
+        if (o.last % 50 == 0) TRY(residual());
+        *last = o.last;
+        *rp = o.rep;
+        return 0;
+    }
+
     int jacobi_resident(double* error)
     {
+        if (chip_jacobi()) {
+            const tl::loop::StopRule rule = stop_rule(0);
+            int last = 0;
+            bool done = false;
+            for (int from = 0;; from = last + 1) {
+                tl::loop::Report rp;
+                TRY(jacobi_chip(from, s.max_iters - from, rule, &last, &rp));
+                TRY(check_report(rp, last, 0));
+                rep->n_jacobi += last - from + 1;
+                *error = rp.err;
+                TRY(confirm(rp, &done));
+                if (done || last + 1 >= s.max_iters) break;
+            }
+            rep->printed_cg_iters = done ? last : s.max_iters;
+            return 0;
+        }
         const size_t bytes = sizeof(double) * (size_t)n;
         TRY(tlhip_copy_device(u_alt, u, bytes));
         int last = 0;

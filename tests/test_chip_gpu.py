@@ -152,3 +152,52 @@ def test_one_iteration_per_launch_is_the_same(hip, size):
     assert out[0][0] == out[1][0]
     for a, b in zip(out[0][1:], out[1][1:]):
         np.testing.assert_array_equal(a, b)
+
+
+def _solver_run(text, dims):
+    from oracle.pyoracle import run_problem
+    from tealeaf_amd.problem import Problem
+    s, states = tdeck.parse_deck(text, dims)
+    want = run_problem(s, states, steps=1, fields=(("u", 3), ("r", 6)))
+    with Problem(s, states) as p:
+        rep = p.step(0)
+        got = {f: p.get(f) for f in ("u", "r")}
+    return s, rep, want["steps"][0], got, {f: a.reshape(s.shape()) for f, a in want["fields"].items()}
+
+
+@pytest.mark.parametrize("sweeps", [1, 51, 53])
+@pytest.mark.parametrize("size", [(40, 30, 0), (65, 129, 0), (517, 200, 0), (1301, 777, 0),
+                                  (33, 32, 9), (127, 90, 60)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_jacobi_bits(hip, oracle, size, sweeps):
+    """No sum feeds back into a sweep, so u and r (the last sweep's input, or
+    the residual of every 50th iteration) are the oracle's bits."""
+    iters = sweeps if size[0] * size[1] < 300000 else min(sweeps, 3)
+    dims = 3 if size[2] else 2
+    text = _text(*size, iters, 2, solver=tdeck.JACOBI).replace("check_result\n", "")
+    s, rep, orep, got, want = _solver_run(text, dims)
+    assert rep["n_jacobi"] == orep["n_jacobi"]
+    np.testing.assert_array_equal(got["u"], want["u"])
+    np.testing.assert_array_equal(got["r"], want["r"])
+    np.testing.assert_allclose(rep["error"], orep["error"], rtol=1e-9)
+
+
+@pytest.mark.parametrize("size,iters", [((40, 30, 0), 70), ((65, 129, 0), 90), ((517, 203, 0), 90),
+                                        ((1301, 777, 0), 45), ((41, 32, 9), 60),
+                                        ((127, 90, 61), 45)],
+                         ids=lambda n: str(n).replace(" ", ""))
+def test_chebyshev_matches_oracle(hip, oracle, size, iters):
+    """From the switch on, Chebyshev iterations have no sums in them; what the
+    two runs differ by is the eigenvalue estimate of the CG steps before, an
+    extreme eigenvalue of a 21 x 21 matrix of their alphas and betas, which
+    moves by no more than they do (1e-12): u to 1e-10."""
+    dims = 3 if size[2] else 2
+    text = _text(*size, iters, 2, solver=tdeck.CHEBY, presteps=20).replace(
+        "epslim = 0.0001", "epslim = 1e30\nerrswitch").replace(
+        "initial_timestep = 0.004", "initial_timestep = 0.4")    # not solved by the CG steps
+    s, rep, orep, got, want = _solver_run(text, dims)
+    assert rep["n_cheby_steps"] == orep["n_cheby_steps"] > 0
+    h = s.halo_depth
+    inner = tuple(slice(h, n - h) for n in s.shape())
+    a, b = got["u"][inner], want["u"][inner]
+    assert np.max(np.abs(a - b)) <= 1e-10 * np.max(np.abs(b))
