@@ -1454,12 +1454,12 @@ int ppcg_inner(int x, int y, int hd, int count, const double* alphas, const doub
                double theta, int init_from_r, const int* neighbours, const double* sd_in,
                double* sd_out, const double* r_in, double* r_out, const double* u_in,
                double* u_out, const double* kx, const double* ky, const double* p,
-               const double* w, unsigned* norm_nb)
+               const double* w, unsigned* norm_nb, bool ring)
 {
     return inner_iterations<double>("tlhip2d_ppcg_inner_iterations", x, y, hd, x, count, alphas,
                                     betas, theta, init_from_r, neighbours, sd_in, sd_out, r_in,
                                     r_out, u_in, u_out, kx, ky, 0.0, p, w,
-                                    p ? loop::alpha() : nullptr, nullptr, true, norm_nb);
+                                    p ? loop::alpha() : nullptr, nullptr, ring, norm_nb);
 }
 
 bool ring_kernel() { return g_fused_variant == 0; }
@@ -1470,11 +1470,11 @@ int ppcg_inner_norm(int x, int y, int hd, int count, const double* alphas, const
                     double theta, int init_from_r, const int* neighbours, const double* sd_in,
                     double* sd_out, const double* r_in, double* r_out, const double* u_in,
                     double* u_out, const double* kx, const double* ky, double alpha,
-                    const double* p, const double* w, double* rrn)
+                    const double* p, const double* w, double* rrn, bool ring)
 {
     return inner_iterations<double>("tlhip2d_ppcg_inner_iterations", x, y, hd, x, count, alphas,
                                     betas, theta, init_from_r, neighbours, sd_in, sd_out, r_in,
-                                    r_out, u_in, u_out, kx, ky, alpha, p, w, nullptr, rrn);
+                                    r_out, u_in, u_out, kx, ky, alpha, p, w, nullptr, rrn, ring);
 }
 
 // calc_p with the loop's beta fused into calc_w, pw finished into alpha.

@@ -833,6 +833,16 @@ extern "C" int tlhip2d_finalise(int x, int y, int hd, double* energy, const doub
 namespace tl {
 namespace loop2d {
 
+int match_ring(int x, int y, int hd, const double* src, double* dst)
+{
+    TL_TRY(tl_ensure_init());
+    const long ring = 2L * hd * x + 2L * hd * (y - 2 * hd);
+    hipLaunchKernelGGL(k_copy_ring2d, dim3(flat_blocks(ring)), dim3(kBlock), 0, tl_stream(),
+                       TlGrid2{x, y, hd}, src, dst);
+    return tl_check_launch("tl2d_copy_ring");
+}
+
+
 int calc_w(int x, int y, int hd, const double* p, double* w, const double* kx, const double* ky)
 {
     const char* what = "tlhip2d_cg_calc_w";

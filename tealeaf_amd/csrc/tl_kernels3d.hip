@@ -1647,15 +1647,21 @@ extern "C" int tlhip_set_pair_rows(int rows)
     return 0;
 }
 
+namespace tl {
+namespace loop3d {
+
+int match_ring(int x, int y, int z, int hd, const double* src, double* dst)
+{
+    TL_TRY(tl_ensure_init());
+    return copy_ring(TlGrid3{x, y, z, hd}, src, dst, "tl3d_copy_ring");
+}
+
 // Two PPCG inner steps per launch; planes per z-tile: tlhip_set_tile_planes
 // when set, else 32 (256^3: 0.384 ms against 0.40 at 16 and 0.46 at 64).
-extern "C" int tlhip3d_ppcg_inner_iterations(int x, int y, int z, int hd, int count,
-                                             const double* alphas, const double* betas,
-                                             const int* neighbours, const double* sd_in,
-                                             double* sd_out, const double* r_in, double* r_out,
-                                             const double* u_in, double* u_out,
-                                             const double* kx, const double* ky,
-                                             const double* kz)
+int ppcg_pair(int x, int y, int z, int hd, int count, const double* alphas, const double* betas,
+              const int* neighbours, const double* sd_in, double* sd_out, const double* r_in,
+              double* r_out, const double* u_in, double* u_out, const double* kx,
+              const double* ky, const double* kz, bool ring)
 {
     const char* what = "tlhip3d_ppcg_inner_iterations";
     TL_TRY(tl_ensure_init());
@@ -1681,9 +1687,11 @@ extern "C" int tlhip3d_ppcg_inner_iterations(int x, int y, int z, int hd, int co
     const int nbz = (int)tl_cdiv(nz, tz);
     const long nb = (long)nwx * nby * nbz;
     if (nb > (1L << 30)) return tl_fail(TLHIP_ERR_ARG, "%s: grid too large", what);
-    TL_TRY(copy_ring(g, sd_in, sd_out, what));
-    TL_TRY(copy_ring(g, r_in, r_out, what));
-    TL_TRY(copy_ring(g, u_in, u_out, what));
+    if (ring) {
+        TL_TRY(copy_ring(g, sd_in, sd_out, what));
+        TL_TRY(copy_ring(g, r_in, r_out, what));
+        TL_TRY(copy_ring(g, u_in, u_out, what));
+    }
     const int slot = tl_timer_begin(what);
 #define TL_PAIR_ARGS nwx, nby, nbz, tz, alphas[0], betas[0], alphas[1], betas[1], sd_in, \
         sd_out, r_in, r_out, u_in, u_out, kx, ky, kz, tl_gate()
@@ -1702,6 +1710,21 @@ extern "C" int tlhip3d_ppcg_inner_iterations(int x, int y, int z, int hd, int co
 #undef TL_PAIR_ARGS
     tl_timer_end(slot);
     return tl_check_launch(what);
+}
+
+}  // namespace loop3d
+}  // namespace tl
+
+extern "C" int tlhip3d_ppcg_inner_iterations(int x, int y, int z, int hd, int count,
+                                             const double* alphas, const double* betas,
+                                             const int* neighbours, const double* sd_in,
+                                             double* sd_out, const double* r_in, double* r_out,
+                                             const double* u_in, double* u_out,
+                                             const double* kx, const double* ky,
+                                             const double* kz)
+{
+    return tl::loop3d::ppcg_pair(x, y, z, hd, count, alphas, betas, neighbours, sd_in, sd_out,
+                                 r_in, r_out, u_in, u_out, kx, ky, kz, true);
 }
 
 // ---------------------------------------------------------------- shared

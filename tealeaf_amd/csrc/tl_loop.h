@@ -122,12 +122,13 @@ int jacobi(int x, int y, int hd, const double* kx, const double* ky, const doubl
 int norm_err(int x, int y, int hd, const double* buf, const loop::StopRule& rule);
 // The fused PPCG launch (calc_ur's alpha from the loop); with norm_nb, the
 // launch also leaves the 2-norm of the r it writes as per-block partials,
-// their count in *norm_nb, for finish_beta.
+// their count in *norm_nb, for finish_beta; ring false: the halo rings of the
+// output buffers are the input's already and are not copied.
 int ppcg_inner(int x, int y, int hd, int count, const double* alphas, const double* betas,
                double theta, int init_from_r, const int* neighbours, const double* sd_in,
                double* sd_out, const double* r_in, double* r_out, const double* u_in,
                double* u_out, const double* kx, const double* ky, const double* p,
-               const double* w, unsigned* norm_nb = nullptr);
+               const double* w, unsigned* norm_nb = nullptr, bool ring = true);
 // Whether the FP64 fused PPCG loop runs the LDS-ring kernel (the one that
 // can form the 2-norm in-launch; tlhip_set_fused_variant).
 bool ring_kernel();
@@ -137,7 +138,9 @@ int ppcg_inner_norm(int x, int y, int hd, int count, const double* alphas, const
                     double theta, int init_from_r, const int* neighbours, const double* sd_in,
                     double* sd_out, const double* r_in, double* r_out, const double* u_in,
                     double* u_out, const double* kx, const double* ky, double alpha,
-                    const double* p, const double* w, double* rrn);
+                    const double* p, const double* w, double* rrn, bool ring = true);
+// The halo ring of src into dst.
+int match_ring(int x, int y, int hd, const double* src, double* dst);
 }  // namespace loop2d
 
 namespace loop3d {
@@ -157,6 +160,13 @@ int calc_ur_cond(int x, int y, int z, int hd, double* u, const double* p, double
 int calc_ur_only(int x, int y, int z, int hd, double* u, const double* p, double* r,
                  const double* w);
 int norm(int x, int y, int z, int hd, const double* buf, const loop::StopRule& rule);
+// The halo ring of src into dst.
+int match_ring(int x, int y, int z, int hd, const double* src, double* dst);
+// tlhip3d_ppcg_inner_iterations, ring as in loop2d::ppcg_inner.
+int ppcg_pair(int x, int y, int z, int hd, int count, const double* alphas, const double* betas,
+              const int* neighbours, const double* sd_in, double* sd_out, const double* r_in,
+              double* r_out, const double* u_in, double* u_out, const double* kx,
+              const double* ky, const double* kz, bool ring);
 int jacobi(int x, int y, int z, int hd, const double* kx, const double* ky, const double* kz,
            const double* u0, const double* u_in, double* u_out, loop::ErrMode mode,
            const loop::StopRule& rule);
