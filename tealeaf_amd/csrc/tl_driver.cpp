@@ -570,19 +570,7 @@ struct tlhip_problem {
 
     int cg_body(const tl::loop::StopRule& rule)
     {
-        if (cond_ok()) {
-            if (pending_p) {
-                pending_p = false;
-                TRY(tl::loop2d::calc_pw_cond(x, y, hd, true, p, p_alt, r, nullptr, cond, rx, ry));
-                std::swap(p, p_alt);
-            } else {
-                TRY(tl::loop2d::calc_pw_cond(x, y, hd, false, p, nullptr, nullptr, nullptr, cond,
-                                             rx, ry));
-            }
-            TRY(tl::loop2d::calc_ur_cond(x, y, hd, u, p, r, cond, rx, ry, rule));
-            pending_p = true;
-            return 0;
-        } else if (cond3_ok()) {
+        if (cond3_ok()) {
             if (pending_p) {
                 pending_p = false;
                 TRY(tl::loop3d::calc_pw_cond(x, y, z, hd, true, p, p_alt, r, nullptr, cond, rx, ry,
