@@ -487,15 +487,17 @@ typedef struct tlhip_problem tlhip_problem;
  * Results are identical either way.  Default on: at 4096^2 on MI355X the
  * fused pass (48 B/cell, 0.162 ms) takes 9% less than the two (0.177 ms). */
 int tlhip_set_cg_fusion(int on);
-/* Whether the driver's CG steps (CG, and the CG phase of Chebyshev and
- * PPCG; 2D and 3D, halo depth >= 2, even x, with tlhip_set_cg_fusion on)
- * run as the cond pair (tlhip2d/3d_cg_calc_pw_cond without storing w, then
- * tlhip2d/3d_cg_calc_ur_cond) and 2D PPCG's calc_p + calc_w reads cond in
- * place of kx and ky.  u, p and r
- * are the reference's expressions either way; rrn is summed in another
- * order, so results agree to rounding.  Default on: at 4096^2 on MI355X a
- * CG step's two passes take 0.284 ms against 0.333 ms (32 + 48 B/cell
- * against 48 + 48).  No counterpart in the reference. */
+/* How the driver's CG steps (CG, and the CG phase of Chebyshev and PPCG;
+ * with tlhip_set_cg_fusion on) run.  On: grids that fit the chip run many
+ * steps to a launch with one meeting of the blocks per step; larger 2D
+ * grids (halo depth >= 2, even x) one pass per step; larger 3D grids the
+ * cond pair (tlhip3d_cg_calc_pw_cond without storing w, then
+ * tlhip3d_cg_calc_ur_cond); and 2D PPCG's calc_p + calc_w reads cond in
+ * place of kx and ky.  The first two predict beta from the sums of the same
+ * meeting or pass and recompute rrn; results agree with those of off to
+ * rounding.  Off: calc_w, calc_ur and calc_p on kx and ky.  Default on: a
+ * CG step takes 0.211 ms against 0.333 ms at 4096^2 on MI355X, 5 us against
+ * 57 us at 512^2.  No counterpart in the reference. */
 int tlhip_set_cg_cond(int on);
 /* Whether the driver runs CG, Jacobi and PPCG outer iterations (2D, 3D)
  * device-resident: alpha = rro/pw, beta = rrn/rro, the
