@@ -155,8 +155,11 @@ struct Mail {           // pinned, host-mapped; armed with TL_MAIL_EMPTY
     double rrn, err, flags, last, alpha, beta;
 };
 
+// part alternates between two buffers by meeting: with one block a wave may
+// start the next meeting while another still reads the last one's parts, and
+// it passes that meeting's barrier only after everybody has.
 struct Shared {
-    double part[kWavesB][kSums];
+    double part[2][kWavesB][kSums];
     double tot[kWavesB][kSums];
     int expired;
 };
@@ -172,7 +175,8 @@ __device__ __forceinline__ bool all_sums(const double v[kSums], Shared& sh, doub
 {
     const int tid = threadIdx.x, lane = tid & (TL_WAVE - 1), wave = tid / TL_WAVE;
     const double c = wave_sum4(v, lane);
-    if ((lane & 15) == 0) sh.part[wave][lane >> 4] = c;
+    double (*part)[kSums] = sh.part[n & 1];
+    if ((lane & 15) == 0) part[wave][lane >> 4] = c;
     double* next = slots + (size_t)((n + 1) % kPhases) * kMaxBlocks * kSums;
     double* mine = slots + (size_t)(n % kPhases) * kMaxBlocks * kSums;
     if (nb > 1 && tid < kSums)
@@ -182,10 +186,10 @@ __device__ __forceinline__ bool all_sums(const double v[kSums], Shared& sh, doub
     __syncthreads();
     double t;
     if (nb == 1) {
-        t = sum_groups(sh.part[lane >> 2][lane & 3]);
+        t = sum_groups(part[lane >> 2][lane & 3]);
     } else {
         if (wave == 0) {
-            const double s = sum_groups(sh.part[lane >> 2][lane & 3]);
+            const double s = sum_groups(part[lane >> 2][lane & 3]);
             if (lane < kSums) st_agent(&mine[blockIdx.x * kSums + lane], s);
         }
         double got = 0.0;

@@ -56,7 +56,9 @@ def _dot(a, b):
 
 def _reference(w, iters, h):
     """u, p, the starting r, r.r after `iters` CG iterations, on the interior,
-    and what other orders of summation can make of alpha (relative, summed)."""
+    what other orders of summation can make of alpha (relative, summed), and
+    how often r.r fell below 1% in an iteration (where its prediction cancels
+    and is not used)."""
     diag = 1.0 + sum(w[c] + np.roll(w[c], -1, axis) for c, axis in
                      zip(("kx", "ky", "kz"), range(w["u0"].ndim - 1, -1, -1)))
     inner = tuple(slice(h, n - h) for n in w["u0"].shape)
@@ -65,7 +67,7 @@ def _reference(w, iters, h):
     r = u - apply_a(w["u0"], *k)
     r0, p = r.copy(), np.zeros_like(w["u0"])
     p[inner] = r
-    rro, slack = _dot(r, r), 0.0
+    rro, slack, cancelled = _dot(r, r), 0.0, 0
     with np.errstate(all="ignore"):
         for _ in range(iters):
             q = apply_a(p, *k)
@@ -76,12 +78,13 @@ def _reference(w, iters, h):
             u += alpha * p[inner]
             r = r - alpha * q
             rrn = _dot(r, r)
+            cancelled += rrn < 0.01 * rro
             p[inner] = np.float64(rrn) / rro * p[inner] + r
             rro = rrn
-    return u, p[inner], r0, rro, slack
+    return u, p[inner], r0, rro, slack, cancelled
 
 
-def _compare(text, dims):
+def _compare(text, dims, cancels=0):
     from oracle.pyoracle import run_problem
     from tealeaf_amd.problem import Problem
     s, states = tdeck.parse_deck(text, dims)
@@ -93,7 +96,8 @@ def _compare(text, dims):
     inner = tuple(slice(h, n - h) for n in s.shape())
     w = {f: a.reshape(s.shape()) for f, a in want["fields"].items()}
     assert rep["n_cg_steps"] == want["steps"][0]["n_cg_steps"]
-    u, p, r0, rr, slack = _reference(w, rep["n_cg_steps"], h)
+    u, p, r0, rr, slack, cancelled = _reference(w, rep["n_cg_steps"], h)
+    assert cancelled >= cancels
     for f, b, start in (("u", u, w["u0"][inner]), ("p", p, r0)):
         a = got[f][inner]
         scale = max(np.max(np.abs(start)), np.max(np.abs(np.nan_to_num(b))))
@@ -130,6 +134,23 @@ GRIDS3 = [(2, 2, 2, 3, 2, False), (64, 16, 8, 5, 2, True), (65, 17, 9, 5, 2, Fal
 def test_cg_3d_matches_reference(hip, oracle, grid):
     nx, ny, nz, iters, hd, recip = grid
     _compare(_text(nx, ny, nz, iters, hd, recip), 3)
+
+
+# nx, ny, nz, timestep, iterations that cancel
+CANCEL = [(48, 48, 0, 4e-5, 4), (48, 48, 0, 4e-4, 2), (64, 128, 0, 4e-5, 6), (2, 2, 2, 0.004, 3),
+          (32, 32, 8, 4e-5, 4), (300, 260, 0, 4e-6, 6), (512, 512, 0, 4e-6, 2),
+          (33, 31, 17, 4e-5, 4)]
+
+
+@pytest.mark.parametrize("case", CANCEL, ids=["x".join(map(str, c[:3])) + f"t{c[3]:g}" for c in CANCEL])
+def test_cancelling_iterations_match_reference(hip, oracle, case):
+    """Short timesteps: r.r falls a hundredfold within an iteration, so the
+    blocks (or the one block's waves) meet a second time for the new r.r,
+    straight after the first meeting."""
+    nx, ny, nz, dt, cancels = case
+    text = _text(nx, ny, nz, 60, 2).replace("initial_timestep = 0.004", f"initial_timestep = {dt}")
+    assert f"initial_timestep = {dt}" in text
+    _compare(text, 3 if nz else 2, cancels)
 
 
 @pytest.mark.parametrize("size", [(40, 30, 0), (300, 260, 0), (40, 33, 21)])
