@@ -204,6 +204,54 @@ def test_driver_3d_pairs_bit_identical(hip, resident, n, inner):
     assert summ == base[3]
 
 
+CHUNK_FIELDS = ("density0", "density", "energy0", "energy", "u", "u0", "p", "r", "mi", "w", "kx",
+                "ky", "kz", "sd", "u_alt", "sd_alt", "volume", "x_area", "y_area", "z_area")
+
+
+@pytest.mark.parametrize("resident", [1, 0])
+@pytest.mark.parametrize("dims", [2, 3])
+def test_refused_candidates_keep_the_rings_equal(hip, resident, dims):
+    """The inner launches swap u with its partner and write interiors only, so
+    both must have the same halo.  With a relative residual below what FP64
+    reaches, the true residual refuses the recurrence's candidates up to
+    max_iters and refreshes u's halo each time; 20 inner steps are an even
+    number of launches, so it is always the same buffer's.  An adopted chunk's
+    buffers are the caller's, who can compare the two."""
+    import ctypes
+
+    from tealeaf_amd.device import DeviceArray
+    from tealeaf_amd.problem import Problem
+    text = (tdeck.layered_2d(90, 1, solver=tdeck.PPCG, presteps=15, inner=20, max_iters=60)
+            if dims == 2 else
+            tdeck.cuboid_3d(24, 1, solver=tdeck.PPCG, presteps=10, inner=20, max_iters=40))
+    s, states = tdeck.parse_deck(text, dims)
+    f = {}
+    with Problem(s, states) as donor:
+        for k in CHUNK_FIELDS:
+            f[k] = (DeviceArray.from_host(donor.get(k)) if k in ("density", "energy0", "energy")
+                    else DeviceArray(donor.n))
+    chunk = (ctypes.c_void_p * len(CHUNK_FIELDS))(*[f[k].ptr for k in CHUNK_FIELDS])
+    cs, handle, rep = tdeck.c_settings(s), ctypes.c_void_p(), tdeck.CStepReport()
+    hip.tlhip_set_resident(resident)
+    try:
+        hip.tlhip_problem_adopt(ctypes.addressof(cs), ctypes.addressof(chunk),
+                                ctypes.addressof(handle))
+        hip.tlhip_problem_set_solve(handle.value, 0, 1e-17)
+        hip.tlhip_problem_step(handle.value, 0, ctypes.addressof(rep))
+    finally:
+        hip.tlhip_set_resident(1)
+        if handle.value:
+            hip.tlhip_problem_destroy(handle.value)
+    assert rep.n_true_residuals >= 3 and rep.n_ppcg_outer > 3
+    halo = np.ones(s.shape(), dtype=bool)
+    halo[tuple(slice(s.halo_depth, -s.halo_depth) for _ in s.shape())] = False
+    u, partner = (f[k].download().reshape(s.shape())[halo] for k in ("u", "u_alt"))
+    assert np.any(u != 0.0)
+    np.testing.assert_array_equal(u, partner)
+    for a in f.values():
+        a.free()
+
+
 def test_set_ppcg_fusion_range(hip):
     assert hip.dll.tlhip_set_ppcg_fusion(11) != 0
     assert hip.dll.tlhip_set_ppcg_fusion(-1) != 0
