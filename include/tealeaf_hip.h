@@ -566,6 +566,11 @@ int tlhip_problem_set_solve(tlhip_problem* p, int precision, double rel_residual
  * of the whole chunk; u, u0, r, p and w are overwritten. */
 int tlhip_problem_adjoint(tlhip_problem* p, int steps, const double* u_target,
         double* loss, double* grad_log_density, tlhip_step_report* reports);
+/* Whether the problem's loops run on the chip where the grid fits it (many
+ * iterations to a launch, fields in registers and LDS; on by default).  Off,
+ * they run as on larger grids, launch by launch: the same iterations to
+ * rounding of CG's sums.  Takes effect at the next timestep. */
+int tlhip_problem_set_on_chip(tlhip_problem* p, int on);
 /* Allocate a chunk on the device and initialise it as
  * 2d/initialise.c:11-31 does (set_chunk_data, set_chunk_state, halo prime,
  * store_energy). */

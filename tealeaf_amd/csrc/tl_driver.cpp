@@ -169,6 +169,7 @@ struct tlhip_problem {
     // sd_alt, r and r_alt (match_rings).
     bool rings_match = false;
     tl::chip::Plan chip;         // tiles of the one-launch loops; ok where the grid fits
+    bool on_chip = true;         // tlhip_problem_set_on_chip
 
     // -------------------------------------------------------- kernels
     int local_halos(int depth)
@@ -363,7 +364,8 @@ struct tlhip_problem {
 
     // CG steps of grids that fit the chip run many to a launch (tl_chip.h).
     // The host-driven loop launches one at a time: the same bits.
-    bool chip_cg() const { return chip.ok && g_cg_cond && g_cg_fusion && interior(); }
+    bool fits_chip() const { return chip.ok && on_chip && interior(); }
+    bool chip_cg() const { return fits_chip() && g_cg_cond && g_cg_fusion; }
 
     int cg_step_chip(int tt, double* rro, double* error)
     {
@@ -380,6 +382,11 @@ struct tlhip_problem {
     }
 
     // 2D CG steps of larger grids: one pass per iteration (tl_cg_pass.h).
+    bool wants_r_alt() const
+    {
+        return dims == 2 && hd >= 2 && s.solver >= 1 && s.solver <= 3 && x % 2 == 0 &&
+               !(chip.ok && on_chip);
+    }
     bool pass_cg() const { return !chip_cg() && cond_ok() && r_alt; }
 
     int cg_pass(bool update, double alpha, double beta, double out[4])
@@ -1133,7 +1140,7 @@ struct tlhip_problem {
     // (tl_chip.h); the reference's own stop test, as fused_cheby.
     bool chip_cheby() const
     {
-        return chip.ok && interior() && rel_tol <= 0.0 && (dims == 2 || s.eps < 1.0);
+        return fits_chip() && rel_tol <= 0.0 && (dims == 2 || s.eps < 1.0);
     }
 
     // Several Chebyshev iterations per pass (2D).  With the relative stop
@@ -1616,7 +1623,7 @@ struct tlhip_problem {
     // 3D with 8 cells per thread: the sweep's division leaves too few
     // registers (128^3: 46 us a sweep against 24 us with the sweep's own
     // launches; 80^3, 4 cells per thread: 6.9 against 14 us).
-    bool chip_jacobi() const { return chip.ok && interior() && !(dims == 3 && chip.k == 8); }
+    bool chip_jacobi() const { return fits_chip() && !(dims == 3 && chip.k == 8); }
 
     // At most count iterations from t0 in one launch (tl_chip.h).  r then
     // holds what the loop leaves there: the last sweep's input, halo included
@@ -1921,6 +1928,15 @@ extern "C" int tlhip_problem_set_solve(tlhip_problem* P, int precision, double r
     return 0;
 }
 
+extern "C" int tlhip_problem_set_on_chip(tlhip_problem* P, int on)
+{
+    if (!P) return tl_fail(TLHIP_ERR_ARG, "tlhip_problem_set_on_chip: null problem");
+    P->on_chip = on != 0;
+    int rc = 0;
+    if (P->wants_r_alt() && !P->r_alt) P->r_alt = dalloc(P->n, &rc);
+    return rc;
+}
+
 extern "C" int tlhip_problem_adjoint(tlhip_problem* P, int steps, const double* u_target,
                                      double* loss, double* grad_log_density,
                                      tlhip_step_report* reports)
@@ -1981,8 +1997,7 @@ void alloc_partners(tlhip_problem* P, int* rc)
     P->chip = tl::chip::plan(P->dims, P->x, P->y, P->z, P->hd);
     // partner of r: the fused PPCG inner loops (2D ring, 3D two-step launch)
     // and the 2D CG passes
-    if (P->s.solver == 3 || (P->dims == 2 && cg && !P->chip.ok && P->x % 2 == 0))
-        P->r_alt = dalloc(P->n, rc);
+    if (P->s.solver == 3 || P->wants_r_alt()) P->r_alt = dalloc(P->n, rc);
 }
 }  // namespace
 

@@ -53,6 +53,11 @@ class Problem:
         instead of the deck's eps."""
         lib().tlhip_problem_set_solve(self.handle, int(precision), float(rel_residual))
 
+    def set_on_chip(self, on: bool) -> None:
+        """Loops of grids that fit the chip in one launch (the default), or
+        launch by launch as on larger grids."""
+        lib().tlhip_problem_set_on_chip(self.handle, int(on))
+
     def adjoint(self, steps: int, target: np.ndarray):
         """Run `steps` timesteps and return (loss, dloss/dln(density), reports)
         for loss = sum over the interior of (u_N - target)^2."""

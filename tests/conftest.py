@@ -37,3 +37,20 @@ def hip():
 def oracle():
     from oracle.pyoracle import load_oracle
     return load_oracle()
+
+
+@pytest.fixture(params=["chip", "launches"])
+def loops(request, monkeypatch):
+    """Driver tests on small grids run both ways that the loops have: on the
+    chip, where such grids run by default, and launch by launch, as larger
+    grids run."""
+    if request.param == "launches":
+        from tealeaf_amd.problem import Problem
+        init = Problem.__init__
+
+        def launches(self, *args, **kw):
+            init(self, *args, **kw)
+            self.set_on_chip(False)
+
+        monkeypatch.setattr(Problem, "__init__", launches)
+    return request.param

@@ -68,6 +68,7 @@ def _r(s):
     return tuple(r)
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("coefficient", [1, 2])
 def test_adjoint_matches_unrolled_autodiff(hip, coefficient):
     steps = 5

@@ -34,6 +34,7 @@ def _fields(s, seed):
                                energy=ENERGY, halo_depth=s.halo_depth)
 
 
+@pytest.mark.usefixtures("loops")
 def test_3d_blocks_match_oracle(hip):
     from oracle.pyoracle import run_problem
     from tealeaf_amd.problem import Problem

@@ -161,6 +161,7 @@ def _run(hip, text, cond, resident):
         hip.tlhip_set_resident(1)
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("solver", ["CG", "CHEBY", "PPCG"])
 def test_driver_cond_pair_agrees(hip, solver):
     """The driver with the cond pair (the default) against kx/ky passes:
@@ -316,6 +317,7 @@ def _run3(hip, text, cond, resident):
         hip.tlhip_set_resident(1)
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("solver", ["CG", "CHEBY", "PPCG"])
 def test_driver_cond3_pair_agrees(hip, solver):
     """3D: the driver with the cond pair (the default) against the kx/ky/kz

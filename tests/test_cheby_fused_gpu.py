@@ -204,6 +204,7 @@ def _run(hip, text, fusion, inject=None):
         hip.tlhip_set_cheby_fusion(10)
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("case", ["layered", "errswitch", "cut_cg", "cut_cheby", "blocks"])
 def test_driver_cheby_fusion_is_bit_identical(hip, case):
     """The driver with fused Chebyshev launches gives the same bits as one

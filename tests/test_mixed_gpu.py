@@ -63,6 +63,7 @@ REL_CASES = [
 ]
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("name,text,dims,blk", REL_CASES, ids=[c[0] for c in REL_CASES])
 def test_fp64_relative_stop_matches_oracle(hip, name, text, dims, blk):
     from oracle.pyoracle import run_problem

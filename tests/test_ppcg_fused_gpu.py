@@ -153,6 +153,7 @@ def _run_fusions(hip, text, fusions, fused_norm, dims=2):
     return res
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("inner", [1, 7, 10, 12])
 def test_driver_fusion_is_bit_identical(hip, inner):
     """The native driver with the fused inner loop gives the same bits as
@@ -181,6 +182,7 @@ def test_driver_fusion_is_bit_identical(hip, inner):
             assert abs(a - b) <= 1e-13 * abs(b), (summ, base[3])
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("resident", [1, 0])
 @pytest.mark.parametrize("n,inner", [(24, 1), (24, 7), (30, 10), (23, 10)])
 def test_driver_3d_pairs_bit_identical(hip, resident, n, inner):

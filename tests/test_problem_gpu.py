@@ -45,6 +45,7 @@ def _compare(steps_a, steps_b, solver):
             assert abs(pa[k] - pb[k]) <= 1, (k, pa, pb)
 
 
+@pytest.mark.usefixtures("loops")
 @pytest.mark.parametrize("name,text", DECKS, ids=[d[0] for d in DECKS])
 def test_native_driver_matches_oracle(hip, name, text):
     from tealeaf_amd.problem import Problem

@@ -14,9 +14,10 @@ and by the error switch, max_iters (in the CG phase and in the PPCG phase),
 the relative-residual stop whose true-residual check can refuse a
 candidate, PPCG inner-step counts whose fused launches leave the ping-pong
 buffers swapped, 3D (sqrt of the error in the stop test; PPCG's outer loop
-resident around step-by-step inner sweeps), and seeded block densities.  The parity of the resident
-path with the reference itself is held by the other driver tests, which run
-with the default.
+resident around step-by-step inner sweeps), and seeded block densities.  Each
+runs on the chip, where host-driven means one iteration per launch, and
+launch by launch.  The parity of the resident path with the reference itself
+is held by the other driver tests, which run with the default.
 """
 import numpy as np
 import pytest
@@ -24,7 +25,53 @@ import pytest
 from tealeaf_amd import blocks
 from tealeaf_amd import deck as tdeck
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("loops")]
+
+
+CHIP_LOOPS = ("tl_chip_cg", "tl_chip_cheby", "tl_chip_jacobi")
+
+
+# What runs launch by launch: 2D even rows, 2D odd rows, 3D
+@pytest.mark.parametrize("text,entries", [
+    (tdeck.layered_2d(64, 1, solver=tdeck.CG, max_iters=3000), ["tl_cg_pass2d"]),
+    (tdeck.layered_2d(63, 1, solver=tdeck.CG, max_iters=3000), ["tlhip2d_cg_calc_ur"]),
+    (tdeck.layered_2d(64, 1, solver=tdeck.CHEBY, presteps=20, max_iters=3000),
+     ["tl_cg_pass2d", "tlhip2d_cheby_iterations"]),
+    (tdeck.layered_2d(63, 1, solver=tdeck.CHEBY, presteps=20, max_iters=3000),
+     ["tlhip2d_cheby_iterate"]),
+    (tdeck.layered_2d(64, 1, solver=tdeck.JACOBI, eps=1e-8, max_iters=300),
+     ["tlhip2d_jacobi_iterate"]),
+    (tdeck.cuboid_3d(20, 1, solver=tdeck.CG, max_iters=2000), ["tlhip3d_cg_calc_ur_cond"]),
+    (tdeck.cuboid_3d(20, 1, solver=tdeck.CHEBY, presteps=10, max_iters=2000),
+     ["tlhip3d_cheby_solver_iterate"]),
+    (tdeck.cuboid_3d(12, 1, solver=tdeck.JACOBI, eps=1e-8, max_iters=300),
+     ["tlhip3d_jacobi_solver_iterate"]),
+], ids=["2d-cg", "2d-cg-odd", "2d-cheby", "2d-cheby-odd", "2d-jacobi", "3d-cg", "3d-cheby",
+        "3d-jacobi"])
+def test_loops_run_where_they_should(hip, loops, text, entries):
+    """The timer's launch counts: the on-chip loops alone, or none of them and
+    the passes that larger grids run."""
+    import ctypes
+    from tealeaf_amd.problem import Problem
+
+    def launches(name):
+        ms, n = ctypes.c_double(), ctypes.c_long()
+        hip.tlhip_kernel_timer_read_entry(name.encode(), ctypes.addressof(ms), ctypes.addressof(n))
+        return n.value
+
+    with Problem.from_deck(text) as p:
+        hip.tlhip_kernel_timer_start(",".join(CHIP_LOOPS + tuple(entries)).encode())
+        try:
+            p.step(0)
+        finally:
+            chip = [launches(k) for k in CHIP_LOOPS]
+            passes = [launches(k) for k in entries]
+            ms, n = ctypes.c_double(), ctypes.c_long()
+            hip.tlhip_kernel_timer_read(ctypes.addressof(ms), ctypes.addressof(n))   # and off
+    if loops == "chip":
+        assert sum(chip) > 0 and sum(passes) <= 1, (chip, passes)   # (Chebyshev's first iteration)
+    else:
+        assert sum(chip) == 0 and all(passes), (chip, passes)
 
 
 def _run(hip, text, resident, dims=None, inject=None, rel=0.0, extra=()):
@@ -65,8 +112,8 @@ def test_2d_layered(hip, solver):
 def test_2d_odd_width(hip, solver):
     """An odd row length (77 + 4 halo cells): one cell per lane, no fused
     calc_p + calc_w and no fused PPCG or Chebyshev loop, so the resident CG
-    body runs calc_w, calc_ur, calc_p and a halo update per iteration, and
-    the PPCG outer loop stays host-driven."""
+    body (launch by launch) runs calc_w, calc_ur, calc_p and a halo update per
+    iteration, and the PPCG outer loop stays host-driven."""
     eps = 1e-8 if solver == tdeck.JACOBI else 1e-15
     _same(hip, tdeck.layered_2d(77, 2, solver=solver, presteps=20, eps=eps, max_iters=3000),
           extra=("r",))
