@@ -998,6 +998,7 @@ struct Host {
     unsigned* rounds = nullptr;
     double* coefs = nullptr;      // [2 * kChunk]
     Mail* mail = nullptr;
+    bool late = false;            // a launch whose report was given up on may still run
     int cus = 0;
 };
 Host g_chip;
@@ -1059,6 +1060,10 @@ int prepare(int nb, size_t xdoubles, const char* what)
 {
     Host& h = g_chip;
     TL_TRY(tl_ensure_init());
+    if (h.late) {       // its report must not be taken for the next launch's
+        CHIP_HIP(hipStreamSynchronize(tl_stream()), what);
+        h.late = false;
+    }
     if (!h.slots) {
         CHIP_HIP(hipMalloc(&h.slots, sizeof(double) * kPhases * kMaxBlocks * kSums), what);
         CHIP_HIP(hipMalloc(&h.rounds, sizeof(unsigned) * kMaxBlocks), what);
@@ -1202,7 +1207,9 @@ int run(const Plan& pl, int count, const char* what, Args&& args, Mail* m)
         CHIP_HIP(hipLaunchCooperativeKernel(fn, dim3(nb), dim3(kThreads), ptrs, (unsigned)lds,
                                             tl_stream()), what);
         tl_timer_end(slot);
+        g_chip.late = true;
         TL_TRY(wait_mail(m, what));
+        g_chip.late = false;
         if (m->flags < 0.0)
             return tl_fail(TLHIP_ERR_HIP, "%s: a block waited over %.0f s for another", what, kWaitS);
         return 0;

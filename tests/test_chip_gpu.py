@@ -222,3 +222,26 @@ def test_chebyshev_matches_oracle(hip, oracle, size, iters):
     inner = tuple(slice(h, n - h) for n in s.shape())
     a, b = got["u"][inner], want["u"][inner]
     assert np.max(np.abs(a - b)) <= 1e-10 * np.max(np.abs(b))
+
+
+def test_late_report_is_not_the_next_launchs(hip):
+    """A wait limit that runs out while a launch is still at work (it ends by
+    itself a few ms later): the step fails, and the next problem's step gets
+    its own report, not the late one."""
+    from tealeaf_amd.abi import TealeafError
+    from tealeaf_amd.problem import Problem
+    slow = _text(1000, 1000, 0, 4000, 2, solver=tdeck.JACOBI)          # 20 ms or more
+    quick = _text(40, 30, 0, 7, 2, solver=tdeck.JACOBI).replace("check_result\n", "")
+    with Problem.from_deck(quick, 2) as q:
+        want = q.step(0), q.get("u")
+    with Problem.from_deck(slow, 2) as p, Problem.from_deck(quick, 2) as q:
+        hip.tlhip_set_wait_limit(1e-4)
+        try:
+            with pytest.raises(TealeafError, match="no report"):
+                p.step(0)
+        finally:
+            hip.tlhip_set_wait_limit(0.0)
+        got = q.step(0), q.get("u")
+    assert want[0]["n_jacobi"] == 7
+    assert got[0] == want[0]
+    np.testing.assert_array_equal(got[1], want[1])
