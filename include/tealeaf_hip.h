@@ -63,7 +63,8 @@ int tlhip_device(void);
 const char* tlhip_last_error(void);
 int tlhip_synchronize(void);
 /* Longest a host-side wait for a device result (a reduction scalar, a
- * resident loop's iteration report) may take before the call fails with
+ * resident loop's iteration report, the report of an on-chip launch, which
+ * runs up to 4096 iterations) may take before the call fails with
  * TLHIP_ERR_HIP and a message naming what it waited for; <= 0 restores
  * the default of 300 s.  No reference counterpart: the reference's
  * drivers block in their device synchronisation. */

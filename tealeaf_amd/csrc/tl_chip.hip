@@ -811,7 +811,9 @@ struct ChebyArgs {
 // Iterations of the Chebyshev loop (2d/drivers/cheby_driver.c with
 // cheby.c:57-85): w = A u, r = u0 - w, p = alpha p + beta r, u += p.  Blocks
 // meet their neighbours only, except where the norm of r is due (every tenth
-// iteration from the estimate on).
+// iteration from the estimate on) and in the launch's last iteration: a block
+// whose wait expired far from block 0, which reports, would otherwise leave
+// its tile behind and go unnoticed.
 template <int DIMS, int K, int LXS>
 __global__ void __launch_bounds__(kThreads) k_chip_cheby(ChebyArgs A)
 {
@@ -844,7 +846,7 @@ __global__ void __launch_bounds__(kThreads) k_chip_cheby(ChebyArgs A)
         double un[K], v[kSums] = {0.0, 0.0, 0.0, 0.0};
         const int t = A.it0 + n;
         const bool norm = A.k0 + n >= A.est && (t + 1) % 10 == 0;
-        const bool keep_r = norm || n + 1 >= A.count;        // it may end here
+        const bool may_end = norm || n + 1 >= A.count;
         const unsigned cell0 = opaque(tl.first);
         co.visit(tl, s_u, s_k, [&](int k, double c, const auto& x, const auto& y, const auto& z) {
             const double r = u0(k, cell0) - co.product(c, x, y, z);
@@ -852,7 +854,7 @@ __global__ void __launch_bounds__(kThreads) k_chip_cheby(ChebyArgs A)
             un[k] = c + p[k];
             if (k < tl.kn) {
                 v[0] += r * r;
-                if (keep_r) A.r[cell0 + k * tl.kstep] = r;
+                if (may_end) A.r[cell0 + k * tl.kstep] = r;
             }
         });
         __syncthreads();          // everybody has read the old u
@@ -862,13 +864,15 @@ __global__ void __launch_bounds__(kThreads) k_chip_cheby(ChebyArgs A)
         double* xb = A.xbuf + (size_t)(n & 1) * tl.xall;
         if (nb > 1) tl.hand_over(un, xb);
         bool fine = true;
-        if (norm) {
+        if (may_end) {
             double tot[kSums];
             fine = all_sums(v, sh, A.slots, meeting++, nb, tot);
-            rrn = tot[0];
-            err = A.sqrt_err ? sqrt(rrn) : rrn;
-            normed = t;
-            if (fabs(err) < A.eps) flags = loop::kConverged;
+            if (norm) {
+                rrn = tot[0];
+                err = A.sqrt_err ? sqrt(rrn) : rrn;
+                normed = t;
+                if (fabs(err) < A.eps) flags = loop::kConverged;
+            }
         } else if (nb > 1) {
             fine = meet_neighbours(g, tl, A.rounds, n + 1, sh);
         }
