@@ -570,7 +570,10 @@ int tlhip_problem_adjoint(tlhip_problem* p, int steps, const double* u_target,
 /* Whether the problem's loops run on the chip where the grid fits it (many
  * iterations to a launch, fields in registers and LDS; on by default).  Off,
  * they run as on larger grids, launch by launch: the same iterations to
- * rounding of CG's sums.  Takes effect at the next timestep. */
+ * rounding of CG's sums.  2: on, with the first launch taken for one that the
+ * runtime refuses because not all blocks can be resident, after which the
+ * problem's loops run launch by launch (a test of that way out).  Takes effect
+ * at the next timestep. */
 int tlhip_problem_set_on_chip(tlhip_problem* p, int on);
 /* Allocate a chunk on the device and initialise it as
  * 2d/initialise.c:11-31 does (set_chunk_data, set_chunk_state, halo prime,

@@ -17,6 +17,7 @@ namespace chip {
 // along x, the others along y.
 struct Plan {
     bool ok = false;
+    bool refuse = false;        // take every launch for refused (tests)
     int dims = 0, x = 0, y = 0, z = 0, hd = 0;
     int k = 0, lxs = 0;
     int tx = 0, ty = 0, tz = 0;
@@ -25,6 +26,11 @@ struct Plan {
 
 // The plan for a grid (halo included), ok = false where it does not fit.
 Plan plan(int dims, int x, int y, int z, int hd);
+
+// Returned by the loops when not all of their blocks can be resident at once
+// (CUs masked from the stream, or a launch the runtime refuses for it):
+// nothing has run and no field has changed.
+constexpr int kRefused = -1;
 
 // What a run of iterations ended with.
 struct Outcome {

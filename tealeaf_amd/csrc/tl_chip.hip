@@ -42,6 +42,7 @@
 #include "tl_lanes.h"
 #include "tealeaf_hip.h"
 
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -1161,6 +1162,8 @@ Plan plan(int dims, int x, int y, int z, int hd)
     Plan best;
     const int nx = x - 2 * hd, ny = y - 2 * hd, nz = dims == 3 ? z - 2 * hd : 1;
     if (nx < 1 || ny < 1 || nz < 1) return best;
+    // (an environment that masks CUs does not show in the device's count)
+    if (getenv("HSA_CU_MASK") || getenv("ROC_GLOBAL_CU_MASK")) return best;
     const int most = std::min(kMaxBlocks, compute_units());
     // A block per CU at most: blocks wait for each other.  The fewest cells
     // per thread that fit are fastest (us per CG iteration with 1, 2, 4, 8
@@ -1189,6 +1192,19 @@ Plan plan(int dims, int x, int y, int z, int hd)
 }
 
 namespace {
+// Whether the stream's CUs hold all blocks at once.
+bool room_for(int blocks)
+{
+    uint32_t mask[32] = {};
+    if (hipExtStreamGetCUMask(tl_stream(), 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    int cus = 0;
+    for (uint32_t m : mask) cus += __builtin_popcount(m);
+    return cus >= blocks;
+}
+
 // Launch one of the loops, args(g) giving its arguments, and wait for its
 // report.
 template <template <int, int, int> class Kernel, class Args>
@@ -1200,6 +1216,7 @@ int run(const Plan& pl, int count, const char* what, Args&& args, Mail* m)
         constexpr int D = decltype(dims)::value, K = decltype(kc)::value;
         constexpr int LXS = decltype(row)::value;
         const int nb = pl.blocks();
+        if (pl.refuse || !room_for(nb)) return kRefused;
         TL_TRY(prepare(nb, 2 * (size_t)nb * faces_of<D, K>(LXS).total(), what));
         const size_t lds = lds_bytes<D, K>(LXS);
         const void* fn = Kernel<D, K, LXS>::fn();
@@ -1208,8 +1225,14 @@ int run(const Plan& pl, int count, const char* what, Args&& args, Mail* m)
         arm_mail();
         void* ptrs[] = {&a};
         const int slot = tl_timer_begin(what);
-        CHIP_HIP(hipLaunchCooperativeKernel(fn, dim3(nb), dim3(kThreads), ptrs, (unsigned)lds,
-                                            tl_stream()), what);
+        const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(nb), dim3(kThreads), ptrs,
+                                                        (unsigned)lds, tl_stream());
+        if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported ||
+            e == hipErrorInvalidConfiguration || e == hipErrorLaunchOutOfResources) {
+            (void)hipGetLastError();
+            return kRefused;
+        }
+        CHIP_HIP(e, what);
         tl_timer_end(slot);
         g_chip.late = true;
         TL_TRY(wait_mail(m, what));

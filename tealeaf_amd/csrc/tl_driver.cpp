@@ -239,19 +239,37 @@ struct tlhip_problem {
         rz = rz_;
         if (dims == 2) {
             TRY(tlhip2d_cg_init(x, y, hd, s.coefficient, rx, ry, rro, density, energy, u, p, r, w, kx, ky));
-            if (cond_ok() && !(chip_cg() && s.solver != 3))
-                TRY(tlhip2d_cg_cond(x, y, hd, s.coefficient, density, cond));
         } else {
             TRY(tlhip3d_cg_solver_init(x, y, z, hd, s.coefficient, rx, ry, rz, rro, density,
                                        energy, u, p, r, w, kx, ky, kz));
-            if (cond3_ok() && !chip_cg())
-                TRY(tlhip3d_cg_cond(x, y, z, hd, s.coefficient, density, cond));
         }
+        TRY(form_cond());
         reset_fields();
         fields[F_U] = fields[F_P] = true;
         TRY(halo_update(1));
         TRY(copy_u());
         return start_solve();
+    }
+
+    // cond where a pass will read it
+    int form_cond()
+    {
+        if (dims == 2 && cond_ok() && !(chip_cg() && s.solver != 3))
+            return tlhip2d_cg_cond(x, y, hd, s.coefficient, density, cond);
+        if (dims == 3 && cond3_ok() && !chip_cg())
+            return tlhip3d_cg_cond(x, y, z, hd, s.coefficient, density, cond);
+        return 0;
+    }
+
+    // An on-chip launch was refused (tl::chip::kRefused): this solve goes on
+    // launch by launch from the fields in hand, and so do later ones.
+    int leave_chip()
+    {
+        chip.ok = false;
+        int rc = 0;
+        if (wants_r_alt() && !r_alt) r_alt = dalloc(n, &rc);
+        TRY(rc);
+        return form_cond();
     }
 
     // -------------------------------------------------------- deferred calc_p
@@ -442,7 +460,11 @@ struct tlhip_problem {
 
     int cg_main_step(int tt, double* rro, double* error)
     {
-        if (chip_cg()) return cg_step_chip(tt, rro, error);
+        if (chip_cg()) {
+            const int rc = cg_step_chip(tt, rro, error);
+            if (rc != tl::chip::kRefused) return rc;
+            TRY(leave_chip());
+        }
         if (pass_cg()) return cg_step_pass(tt, rro, error);
         double alpha = 0.0, rrn = 0.0;
         if (cond_ok()) {
@@ -893,7 +915,11 @@ struct tlhip_problem {
         const tl::loop::StopRule rule = stop_rule(sw);
         tl::chip::Outcome o{};
         for (int from = t0;; from = o.last + 1) {
-            TRY(tl::chip::cg(chip, u, p, r, kx, ky, kz, from, s.max_iters - from, rule, &o));
+            const int rc = tl::chip::cg(chip, u, p, r, kx, ky, kz, from, s.max_iters - from, rule, &o);
+            if (rc == tl::chip::kRefused && from > t0)
+                return tl_fail(TLHIP_ERR_HIP, "resident loop: no room on the chip for the launch of "
+                               "iteration %d", from);
+            TRY(rc);
             TRY(check_report(o.rep, o.last, sw));
             if (o.rep.flags || o.last + 1 >= s.max_iters) break;
         }
@@ -928,15 +954,21 @@ struct tlhip_problem {
                     continue;
                 }
             }
-            if (chip_cg())
-                TRY(cg_run_chip(from, sw, rro, error, &last, &rp));
-            else
+            if (chip_cg()) {
+                const int rc = cg_run_chip(from, sw, rro, error, &last, &rp);
+                if (rc == tl::chip::kRefused) {
+                    TRY(leave_chip());
+                    continue;
+                }
+                TRY(rc);
+            } else {
                 TRY(run_resident(from, sw, true,
                                  [&](const tl::loop::StopRule& rule, int j) {
                                      return pass_cg() ? cg_body_pass(rule, j, from)
                                                       : cg_body(rule);
                                  },
                                  rro, error, &last, &rp, true, can_defer_p() || cond3_ok()));
+            }
             have_sums = false;
             rep->n_cg_steps += last - from + 1;
             *tt = last;
@@ -1079,24 +1111,9 @@ struct tlhip_problem {
                 TRY(halo_update(1));
                 TRY(cheby_step(ncheby, true, error));
                 est = est_iterations(*error, bb);
-            } else if (chip_cheby()) {
-                // all the iterations up to the stop in one launch (one per
-                // launch without fusion)
-                const int from = tt;
-                tl::chip::Outcome o;
-                TRY(tl::chip::cheby(chip, u, p, r, u0, kx, ky, kz, tt,
-                                    g_cheby_fusion > 1 ? s.max_iters - tt : 1, ncheby, est,
-                                    &cheby_alphas[ncheby], &cheby_betas[ncheby], s.eps, dims == 3,
-                                    &o));
-                rep->n_cheby_steps += o.last - from + 1;
-                ncheby += o.last - from;
-                tt = o.last;
-                const int normed = (int)o.alpha;
-                if (normed >= 0) *error = o.rep.rrn;
-                // 3D takes the root of the error at every iteration's test,
-                // whether that iteration formed it or not
-                if (dims == 3)
-                    for (int j = normed >= 0 ? normed : from; j < tt; ++j) *error = std::sqrt(*error);
+            } else if (int rc; chip_cheby() && (rc = cheby_on_chip(&tt, &ncheby, est, error)) !=
+                                                   tl::chip::kRefused) {
+                TRY(rc);
             } else if (fused_cheby()) {
                 // Iterations tt, tt+1, ... in one pass, up to and including
                 // the next one that computes the norm (the only ones after
@@ -1141,6 +1158,30 @@ struct tlhip_problem {
     bool chip_cheby() const
     {
         return fits_chip() && rel_tol <= 0.0 && (dims == 2 || s.eps < 1.0);
+    }
+
+    // All the iterations from *tt up to the stop in one launch (one per launch
+    // without fusion); *tt and *k, the iteration and its coefficient, become
+    // the last one's.
+    int cheby_on_chip(int* tt, int* k, int est, double* error)
+    {
+        const int from = *tt;
+        tl::chip::Outcome o;
+        const int rc = tl::chip::cheby(chip, u, p, r, u0, kx, ky, kz, from,
+                                       g_cheby_fusion > 1 ? s.max_iters - from : 1, *k, est,
+                                       &cheby_alphas[*k], &cheby_betas[*k], s.eps, dims == 3, &o);
+        if (rc == tl::chip::kRefused) TRY(leave_chip());
+        TRY(rc);
+        rep->n_cheby_steps += o.last - from + 1;
+        *k += o.last - from;
+        *tt = o.last;
+        const int normed = (int)o.alpha;
+        if (normed >= 0) *error = o.rep.rrn;
+        // 3D takes the root of the error at every iteration's test,
+        // whether that iteration formed it or not
+        if (dims == 3)
+            for (int j = normed >= 0 ? normed : from; j < o.last; ++j) *error = std::sqrt(*error);
+        return 0;
     }
 
     // Several Chebyshev iterations per pass (2D).  With the relative stop
@@ -1588,13 +1629,17 @@ struct tlhip_problem {
                 never.eps = -1.0;
                 int last;
                 tl::loop::Report rp;
-                TRY(jacobi_chip(tt, 1, never, &last, &rp));
-                rep->n_jacobi++;
-                *error = rp.rrn;
-                bool done;
-                TRY(stop(error, &done));
-                if (done) break;
-                continue;
+                const int rc = jacobi_chip(tt, 1, never, &last, &rp);
+                if (rc != tl::chip::kRefused) {
+                    TRY(rc);
+                    rep->n_jacobi++;
+                    *error = rp.rrn;
+                    bool done;
+                    TRY(stop(error, &done));
+                    if (done) break;
+                    continue;
+                }
+                TRY(leave_chip());
             }
             if (dims == 2) TRY(tlhip2d_jacobi_iterate(x, y, hd, error, kx, ky, u0, u, r));
             else TRY(tlhip3d_jacobi_solver_iterate(x, y, z, hd, error, kx, ky, kz, u0, u, r));
@@ -1656,7 +1701,15 @@ struct tlhip_problem {
             bool done = false;
             for (int from = 0;; from = last + 1) {
                 tl::loop::Report rp;
-                TRY(jacobi_chip(from, s.max_iters - from, rule, &last, &rp));
+                const int rc = jacobi_chip(from, s.max_iters - from, rule, &last, &rp);
+                if (rc == tl::chip::kRefused && from == 0) {
+                    TRY(leave_chip());
+                    return jacobi_resident(error);
+                }
+                if (rc == tl::chip::kRefused)
+                    return tl_fail(TLHIP_ERR_HIP, "resident loop: no room on the chip for the "
+                                   "launch of iteration %d", from);
+                TRY(rc);
                 TRY(check_report(rp, last, 0));
                 rep->n_jacobi += last - from + 1;
                 *error = rp.err;
@@ -1932,6 +1985,7 @@ extern "C" int tlhip_problem_set_on_chip(tlhip_problem* P, int on)
 {
     if (!P) return tl_fail(TLHIP_ERR_ARG, "tlhip_problem_set_on_chip: null problem");
     P->on_chip = on != 0;
+    P->chip.refuse = on == 2;
     int rc = 0;
     if (P->wants_r_alt() && !P->r_alt) P->r_alt = dalloc(P->n, &rc);
     return rc;

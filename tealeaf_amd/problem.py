@@ -53,9 +53,10 @@ class Problem:
         instead of the deck's eps."""
         lib().tlhip_problem_set_solve(self.handle, int(precision), float(rel_residual))
 
-    def set_on_chip(self, on: bool) -> None:
-        """Loops of grids that fit the chip in one launch (the default), or
-        launch by launch as on larger grids."""
+    def set_on_chip(self, on: int) -> None:
+        """Loops of grids that fit the chip in one launch (True, the default),
+        or launch by launch as on larger grids (False); 2: the first on-chip
+        launch is taken for refused."""
         lib().tlhip_problem_set_on_chip(self.handle, int(on))
 
     def adjoint(self, steps: int, target: np.ndarray):

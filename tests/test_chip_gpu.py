@@ -245,3 +245,56 @@ def test_late_report_is_not_the_next_launchs(hip):
     assert want[0]["n_jacobi"] == 7
     assert got[0] == want[0]
     np.testing.assert_array_equal(got[1], want[1])
+
+
+REFUSED = [("2d-cg", _text(64, 50, 0, 400, 2), 2, 1),
+           ("2d-cg-odd", _text(63, 50, 0, 400, 2), 2, 1),
+           ("2d-cheby", _text(64, 50, 0, 400, 2, solver=tdeck.CHEBY), 2, 1),
+           ("2d-cheby-late", _text(64, 50, 0, 400, 2, solver=tdeck.CHEBY), 2, 0),
+           ("2d-cheby-odd-late", _text(63, 50, 0, 400, 2, solver=tdeck.CHEBY), 2, 0),
+           ("2d-ppcg", _text(64, 50, 0, 400, 2, solver=tdeck.PPCG), 2, 1),
+           ("2d-jacobi", _text(64, 50, 0, 60, 2, solver=tdeck.JACOBI), 2, 1),
+           ("3d-cg", _text(20, 18, 16, 400, 2), 3, 1),
+           ("3d-cheby-late", _text(20, 18, 16, 400, 2, solver=tdeck.CHEBY, presteps=10), 3, 0),
+           ("3d-jacobi", _text(20, 18, 16, 60, 2, solver=tdeck.JACOBI), 3, 1)]
+
+
+@pytest.mark.parametrize("resident", [1, 0])
+@pytest.mark.parametrize("name,text,dims,cond", REFUSED, ids=[c[0] for c in REFUSED])
+def test_refused_launch_goes_on_launch_by_launch(hip, name, text, dims, cond, resident):
+    """A launch that the runtime refuses (here: taken for refused) changes
+    nothing, and the solve runs as one that never tried: the same bits over two
+    steps.  Without the cond passes CG does not run on the chip, so the first
+    launch refused is Chebyshev's."""
+    from tealeaf_amd.problem import Problem
+    out = []
+    hip.tlhip_set_resident(resident)
+    hip.tlhip_set_cg_cond(cond)
+    try:
+        for on in (0, 2):
+            with Problem.from_deck(text, dims) as p:
+                p.set_on_chip(on)
+                out.append(([p.step(t) for t in range(2)], [p.get(f) for f in ("u", "r", "energy")]))
+    finally:
+        hip.tlhip_set_resident(1)
+        hip.tlhip_set_cg_cond(1)
+    assert out[0][0] == out[1][0]
+    for a, b in zip(out[0][1], out[1][1]):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("variable", ["HSA_CU_MASK", "ROC_GLOBAL_CU_MASK"])
+def test_masked_cus_keep_off_the_chip(hip, monkeypatch, variable):
+    """An environment that masks CUs (read here when a problem is created; the
+    runtime has read its own long before) leaves no plan for the chip."""
+    import ctypes
+    from tealeaf_amd.problem import Problem
+    monkeypatch.setenv(variable, "0x1")
+    ms, n = ctypes.c_double(), ctypes.c_long()
+    with Problem.from_deck(_text(64, 50, 0, 400, 2), 2) as p:
+        hip.tlhip_kernel_timer_start(b"tl_chip_cg")
+        try:
+            rep = p.step(0)
+        finally:
+            hip.tlhip_kernel_timer_read(ctypes.addressof(ms), ctypes.addressof(n))
+    assert n.value == 0 and rep["n_cg_steps"] > 0
