@@ -28,7 +28,8 @@ __host__ __device__ inline bool scalars(const double s[4], double* alpha, double
     return !(next < 0.01 * s[kRR]);
 }
 
-// Whether a 2D grid can take the pass (the cond pair's conditions).
+// Whether a 2D grid can take the pass (the cond pair's conditions, and room
+// for the partial sums of every strip).
 bool fits2d(int x, int y, int hd);
 
 // The host's form: with update, one iteration's pass (r_in, p_in -> r_out,

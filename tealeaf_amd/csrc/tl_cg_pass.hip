@@ -174,8 +174,8 @@ int launch2d(const char* what, int x, int y, int hd, bool update, double alpha, 
 {
     TL_TRY(tl_ensure_init());
     if (!fits2d(x, y, hd))
-        return tl_fail(TLHIP_ERR_ARG, "%s: needs halo depth >= 2 and an even x (x=%d y=%d hd=%d)",
-                       what, x, y, hd);
+        return tl_fail(TLHIP_ERR_ARG, "%s: needs halo depth >= 2, an even x and at most %d strips "
+                       "of columns (x=%d y=%d hd=%d)", what, TL_MAX_RED_BLOCKS, x, y, hd);
     TL_REQUIRE(r_in && p_in && cond && (!update || (u && r_out && p_out)), what, "null field");
     TL_REQUIRE(!update || (r_out != r_in && p_out != p_in && r_out != p_out && u != r_in &&
                            u != p_in && u != r_out && u != p_out),
@@ -204,7 +204,10 @@ const char* const kName2 = "tl_cg_pass2d";
 
 bool fits2d(int x, int y, int hd)
 {
-    return hd >= 2 && x % 2 == 0 && x > 2 * hd && y > 2 * hd && (long)x * y <= (1L << 31) - 1;
+    if (hd < 2 || x % 2 || x <= 2 * hd || y <= 2 * hd || (long)x * y > (1L << 31) - 1) return false;
+    // one block, with its partial sums, per strip at the least (8.1 million columns)
+    const PitchGrid g{x, hd, x - 2 * hd, y - 2 * hd};
+    return strip_tile<double>(g, 2, g.ny, 1).nbx <= TL_MAX_RED_BLOCKS;
 }
 
 int step2d(int x, int y, int hd, bool update, double alpha, double beta, double* u,

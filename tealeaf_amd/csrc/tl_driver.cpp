@@ -402,10 +402,13 @@ struct tlhip_problem {
     // 2D CG steps of larger grids: one pass per iteration (tl_cg_pass.h).
     bool wants_r_alt() const
     {
-        return dims == 2 && hd >= 2 && s.solver >= 1 && s.solver <= 3 && x % 2 == 0 &&
+        return dims == 2 && s.solver >= 1 && s.solver <= 3 && tl::pass::fits2d(x, y, hd) &&
                !(chip.ok && on_chip);
     }
-    bool pass_cg() const { return !chip_cg() && cond_ok() && r_alt; }
+    bool pass_cg() const
+    {
+        return !chip_cg() && cond_ok() && r_alt && tl::pass::fits2d(x, y, hd);
+    }
 
     int cg_pass(bool update, double alpha, double beta, double out[4])
     {

@@ -47,3 +47,29 @@ def test_host_driven_is_the_same(hip, solver):
     assert out[0][0] == out[1][0]
     for a, b in zip(out[0][1:], out[1][1:]):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("nx,fits", [(65536 * 124, True), (65536 * 124 + 2, False)])
+def test_widest_grids(hip, nx, fits):
+    """A strip of columns needs a block of its own and a place for its partial
+    sums: one strip more than there are places takes the passes over kx and
+    ky.  The same u either way (a timestep that makes the operator well
+    conditioned along x)."""
+    import ctypes
+    from tealeaf_amd.problem import Problem
+    text = _text(nx, 1, 0, 3, 2).replace("initial_timestep = 0.004", "initial_timestep = 1.5e-12")
+    assert "1.5e-12" in text
+    out, ms, n = [], ctypes.c_double(), ctypes.c_long()
+    try:
+        for cond in (1, 0):
+            hip.tlhip_set_cg_cond(cond)
+            with Problem.from_deck(text, 2) as p:
+                hip.tlhip_kernel_timer_start(b"tl_cg_pass2d")
+                rep = p.step(0)
+                hip.tlhip_kernel_timer_read(ctypes.addressof(ms), ctypes.addressof(n))
+                assert rep["n_cg_steps"] == 3
+                assert (n.value > 0) == (fits and cond == 1)
+                out.append(p.get("u"))
+    finally:
+        hip.tlhip_set_cg_cond(1)
+    assert np.max(np.abs(out[0] - out[1])) <= 1e-12 * np.max(np.abs(out[1]))
