@@ -16,16 +16,23 @@ namespace pass {
 // The sums of a pass, in this order.
 enum : int { kPQ, kQQ, kRQ, kRR };
 
+// Whether the r.r after an iteration can be predicted: not where it falls
+// below 1% of the one before, as the terms of the prediction then cancel.
+__host__ __device__ inline bool predictable(double next, double rr)
+{
+    return !(next < 0.01 * rr);
+}
+
 // alpha = r.r / p.q; beta from the predicted r.r of the next iteration.
-// False where the prediction cancels (below 1% of r.r: its error could pass
-// 1e-13): that iteration has to sum the new r.r, two sums a pass apart.
+// False where the prediction cancels: that iteration has to sum the new r.r,
+// two sums a pass apart.
 __host__ __device__ inline bool scalars(const double s[4], double* alpha, double* beta)
 {
     const double a = s[kRR] / s[kPQ];
     const double next = (s[kRR] - 2.0 * a * s[kRQ]) + a * a * s[kQQ];
     *alpha = a;
     *beta = next / s[kRR];
-    return !(next < 0.01 * s[kRR]);
+    return predictable(next, s[kRR]);
 }
 
 // Whether a 2D grid can take the pass (the cond pair's conditions, and room
@@ -43,7 +50,7 @@ int step2d(int x, int y, int hd, bool update, double alpha, double beta, double*
 namespace loop {
 // The sums of a pass finished on the device: the iteration's rrn, beta log,
 // stop rule and report, and the next iteration's alpha, beta and alpha log.
-// Where those cancel, the report carries kCancel and the loop ends.
+// Where those cancel, the report carries kTurn and the loop ends.
 int finish_pass(unsigned nblocks, const StopRule& rule, const char* what);
 // After begin(), before the first pass: the sums of the state it starts from.
 int start_pass(int j0, const double sums[4]);

@@ -165,6 +165,9 @@ struct tlhip_problem {
     // anything else touched them.
     bool have_sums = false;
     double sums[4] = {};
+    // CG of a grid that can take passes runs with two sums an iteration (from
+    // the start of a solve, and again once a prediction has cancelled).
+    bool two_sums = true, cancelled = false;
     // PPCG's inner launches rely on equal halo rings of u and u_alt, sd and
     // sd_alt, r and r_alt (match_rings).
     bool rings_match = false;
@@ -428,22 +431,33 @@ struct tlhip_problem {
         return 0;
     }
 
+    // A solve of such a grid takes its first iteration with two sums (the cond
+    // pair) and goes over to passes after an iteration whose r.r a pass could
+    // have predicted; where a pass's prediction cancels, it goes back to the
+    // pair for good.  So a solve that converges a hundredfold in every
+    // iteration runs the pair throughout.
+    int to_passes()
+    {
+        two_sums = false;
+        have_sums = false;
+        return flush_p();
+    }
+
     int cg_step_pass(int tt, double* rro, double* error)
     {
-        TRY(need_sums());
         double alpha, beta, rrn = 0.0;
-        if (tl::pass::scalars(sums, &alpha, &beta)) {
+        if (!two_sums) TRY(need_sums());
+        if (!two_sums && tl::pass::scalars(sums, &alpha, &beta)) {
             const double old = sums[tl::pass::kRR];
             TRY(cg_pass(true, alpha, beta, sums));
             rrn = sums[tl::pass::kRR];
             beta = rrn / old;
         } else {
-            // the prediction cancels: two sums, a pass apart
-            double old = sums[tl::pass::kRR];
-            have_sums = false;
-            TRY(cg_step_cond(&old, &alpha, &rrn));
-            beta = rrn / old;
-            TRY(calc_p(beta));
+            if (!two_sums) two_sums = cancelled = true;
+            TRY(cg_step_cond(rro, &alpha, &rrn));
+            beta = rrn / *rro;
+            TRY(calc_p_deferred(beta));
+            if (!cancelled && tl::pass::predictable(rrn, *rro)) TRY(to_passes());
         }
         cg_alphas[tt] = alpha;
         cg_betas[tt] = beta;
@@ -540,6 +554,8 @@ struct tlhip_problem {
     {
         bb = 0.0;
         have_sums = false;
+        two_sums = true;
+        cancelled = false;
         rings_match = false;
         if (rel_tol > 0.0 || precision == 1) TRY(norm2(u0, &bb));
         return 0;
@@ -584,7 +600,7 @@ struct tlhip_problem {
         if (conv) want |= tl::loop::kConverged;
         if (sw && switch_now(0, j + 1, err)) want |= tl::loop::kSwitch;
         const bool same_err = err == rp.err || (err != err && rp.err != rp.err);
-        if (want != (rp.flags & ~tl::loop::kCancel) || !same_err)
+        if (want != (rp.flags & ~tl::loop::kTurn) || !same_err)
             return tl_fail(TLHIP_ERR_SOLVER,
                            "resident loop: device report of iteration %d differs from the host's "
                            "test (flags %d, host %d)", j, rp.flags, want);
@@ -607,7 +623,19 @@ struct tlhip_problem {
 
     int cg_body(const tl::loop::StopRule& rule)
     {
-        if (cond3_ok()) {
+        if (cond_ok()) {
+            if (pending_p) {
+                pending_p = false;
+                TRY(tl::loop2d::calc_pw_cond(x, y, hd, true, p, p_alt, r, nullptr, cond, rx, ry));
+                std::swap(p, p_alt);
+            } else {
+                TRY(tl::loop2d::calc_pw_cond(x, y, hd, false, p, nullptr, nullptr, nullptr, cond,
+                                             rx, ry));
+            }
+            TRY(tl::loop2d::calc_ur_cond(x, y, hd, u, p, r, cond, rx, ry, rule));
+            pending_p = true;
+            return 0;
+        } else if (cond3_ok()) {
             if (pending_p) {
                 pending_p = false;
                 TRY(tl::loop3d::calc_pw_cond(x, y, z, hd, true, p, p_alt, r, nullptr, cond, rx, ry,
@@ -822,7 +850,8 @@ struct tlhip_problem {
 
     template <class Body>
     int run_resident(int t0, int sw, bool cg, Body&& body, double* rro, double* error, int* last,
-                     tl::loop::Report* out, bool periodic = true, bool halo_after = false)
+                     tl::loop::Report* out, bool periodic = true, bool halo_after = false,
+                     bool turn = false)
     {
         if (t0 < 0 || t0 >= s.max_iters)
             return tl_fail(TLHIP_ERR_ARG, "resident loop: no iteration to run from %d", t0);
@@ -836,16 +865,21 @@ struct tlhip_problem {
                 tl::loop::end();
             }
         } close;
-        const tl::loop::StopRule rule = stop_rule(sw);
+        tl::loop::StopRule rule = stop_rule(sw);
+        rule.turn = turn;
         // Small grids replay pairs of iterations from a graph after the
         // first iteration (which may differ: calc_w before calc_pw).
         bool graph = periodic && g_graphs && n <= kGraphCells && !tl_timer_active();
         int g0 = -1;
         Ptrs gmid{}, gstart{};
         int next = t0, chk = t0;
+        // A turn is expected at the first report: little is enqueued behind it
+        // (grids that turn are large; one iteration ahead keeps them busy).
+        const int ahead = turn ? 1 : tl::loop::kAhead;
+        double before = *rro;         // rrn of the iteration before chk
         tl::loop::Report rp{};
         for (;;) {
-            while (next < s.max_iters && next <= chk + tl::loop::kAhead) {
+            while (next < s.max_iters && next <= chk + ahead) {
                 if (graph && g0 < 0 && next > t0 && next + 2 <= s.max_iters) {
                     bool ok;
                     gstart = ptrs();
@@ -868,6 +902,7 @@ struct tlhip_problem {
             TRY(tl::loop::wait(chk, &rp));
             TRY(check_report(rp, chk, sw));
             if (rp.flags || chk + 1 >= s.max_iters) break;
+            before = rp.rrn;
             ++chk;
         }
         const Ptrs& q = snap[chk % kSnap];
@@ -879,12 +914,11 @@ struct tlhip_problem {
             tl::loop::end();
             TRY(halo_update(1));
         }
-        if (cg) TRY(tl::loop::logs(t0, chk - t0 + 1, &cg_alphas[t0], &cg_betas[t0]));
-        if (pending_p) {
-            // the last iteration's calc_p waits with its beta (host copy for flush_p)
-            double a;
-            TRY(tl::loop::logs(chk, 1, &a, &pending_beta));
-        }
+        // (read by the eigenvalue estimate only)
+        if (cg && s.solver != 1)
+            TRY(tl::loop::logs(t0, chk - t0 + 1, &cg_alphas[t0], &cg_betas[t0]));
+        // the last iteration's calc_p waits with its beta (host copy for flush_p)
+        if (pending_p) pending_beta = rp.rrn / before;
         *last = chk;
         *out = rp;
         *rro = rp.rrn;
@@ -945,16 +979,13 @@ struct tlhip_problem {
         for (int from = t0;;) {
             int last;
             tl::loop::Report rp{};
-            if (pass_cg()) {
+            bool pass = pass_cg() && !two_sums;
+            if (pass) {
                 TRY(need_sums());
                 double a, b;
                 if (!tl::pass::scalars(sums, &a, &b)) {
-                    TRY(cg_step_pass(from, rro, error));
-                    TRY(halo_update(1));
-                    TRY(stop(error, done));
-                    *tt = from++;
-                    if (*done || from >= s.max_iters || (sw && switch_now(0, from, *error))) return 0;
-                    continue;
+                    two_sums = cancelled = true;
+                    pass = false;
                 }
             }
             if (chip_cg()) {
@@ -965,12 +996,17 @@ struct tlhip_problem {
                 }
                 TRY(rc);
             } else {
+                const bool turn = pass_cg() && !pass && !cancelled;
                 TRY(run_resident(from, sw, true,
                                  [&](const tl::loop::StopRule& rule, int j) {
-                                     return pass_cg() ? cg_body_pass(rule, j, from)
-                                                      : cg_body(rule);
+                                     return pass ? cg_body_pass(rule, j, from) : cg_body(rule);
                                  },
-                                 rro, error, &last, &rp, true, can_defer_p() || cond3_ok()));
+                                 rro, error, &last, &rp, true, can_defer_p() || cond3_ok(),
+                                 turn));
+                if (rp.flags & tl::loop::kTurn) {
+                    if (pass) two_sums = cancelled = true;
+                    else TRY(to_passes());
+                }
             }
             have_sums = false;
             rep->n_cg_steps += last - from + 1;

@@ -1,6 +1,6 @@
 // Shared pieces of the temporally blocked 2D loops (tl_fused2d.hip: the
 // register-window kernels, the Chebyshev loop and the host entry points;
-// tl_ppcg_ring.h: the PPCG loop with its coefficient rows in LDS).
+// tl_ppcg_ring.hip: the PPCG loop with its coefficient rows in LDS).
 #pragma once
 
 #include "tl_lanes.h"
@@ -64,7 +64,7 @@ extern int g_fused_variant;
 extern double g_ring_fill;
 
 // The PPCG loop with the coefficient rows in per-wave LDS rings
-// (tl_ppcg_ring.h); count 1..kMaxFused, mode 0..2 as FusedArgs.  Mode 3
+// (tl_ppcg_ring.hip); count 1..kMaxFused, mode 0..2 as FusedArgs.  Mode 3
 // runs the Chebyshev loop the same way (2d/drivers/cheby_driver.c turns:
 // mirror of u, r = u0 - A u, p = alpha_k p + beta_k r, u += p) with the
 // fields in the PPCG roles: sd_in/sd_out = u, r_in = u0, u_in/u_out = p,

@@ -1492,9 +1492,10 @@ int calc_pw(int x, int y, int hd, const double* p_in, double* p_out, const doubl
     return loop::finish_alpha(nb, what);
 }
 
-// calc_pw_cond in a resident loop (beta from the loop with update; w
-// written unless null) with pw finished into alpha.  p_out's halo is left as
-// calc_pw leaves it.
+// The cond pair in a resident loop: calc_pw_cond (beta from the loop with
+// update; w written unless null) with pw finished into alpha, and
+// calc_ur_cond (alpha from the loop) with rrn finished into beta and the
+// stop rule.  p_out's halo is left as calc_pw leaves it.
 int calc_pw_cond(int x, int y, int hd, bool update, const double* p_in, double* p_out,
                  const double* r, double* w, const double* cond, double rx, double ry)
 {
@@ -1503,6 +1504,15 @@ int calc_pw_cond(int x, int y, int hd, bool update, const double* p_in, double* 
     TL_TRY(launch_pw_cond(what, x, y, hd, update, 0.0, update ? loop::beta() : nullptr, p_in,
                           p_out, r, w, cond, rx, ry, &nb, false));
     return loop::finish_alpha(nb, what);
+}
+
+int calc_ur_cond(int x, int y, int hd, double* u, const double* p, double* r, const double* cond,
+                 double rx, double ry, const loop::StopRule& rule)
+{
+    const char* what = "tlhip2d_cg_calc_ur_cond";
+    unsigned nb = 0;
+    TL_TRY(launch_ur_cond(what, x, y, hd, 0.0, loop::alpha(), u, p, r, cond, rx, ry, &nb));
+    return loop::finish_beta(nb, rule, what);
 }
 
 }  // namespace loop2d

@@ -107,11 +107,11 @@ k_loop_beta(unsigned nblocks, const double* __restrict__ partials, State* st, do
     tl_sum_partials<1>(nblocks, partials, tot);
     if (threadIdx.x != 0) return;
     const double rrn = tot[0];
-    const double b = rrn / st->rro;
+    const double old = st->rro, b = rrn / old;
     st->beta = b;
     blog[j] = b;
     st->rro = rrn;
-    test_and_report(st, ring, j, rrn, rule);
+    test_and_report(st, ring, j, rrn, rule, rule.turn && pass::predictable(rrn, old) ? kTurn : 0);
 }
 
 __global__ void __launch_bounds__(64)
@@ -141,7 +141,7 @@ k_loop_pass(unsigned nblocks, const double* __restrict__ partials, State* st, do
     st->rro = rrn;
     const bool fine = pass::scalars(s, &st->alpha, &st->beta);
     if (j + 1 < cap) alog[j + 1] = st->alpha;
-    test_and_report(st, ring, j, rrn, rule, fine ? 0 : kCancel);
+    test_and_report(st, ring, j, rrn, rule, fine ? 0 : kTurn);
 }
 
 // The Jacobi error of iteration j: assigned (jacobi.c:99) or, for the
