@@ -1166,10 +1166,13 @@ Plan plan(int dims, int x, int y, int z, int hd)
     if (getenv("HSA_CU_MASK") || getenv("ROC_GLOBAL_CU_MASK")) return best;
     const int most = std::min(kMaxBlocks, compute_units());
     // A block per CU at most: blocks wait for each other.  The fewest cells
-    // per thread that fit are fastest (us per CG iteration with 1, 2, 4, 8
-    // cells: 512^2 5.6 5.5 6.1 8.5; 1024^2 - - 7.3 9.7; 64^3 - 8.5 9.4 17.2),
-    // except that a grid which fits one block needs no meeting across the
-    // chip (48^2, one block 3.7 us a sweep, several 4.3).
+    // per thread that fit are fastest or nearly so (us per CG iteration with 1,
+    // 2, 4, 8 cells: 300 x 260 4.2 4.6 5.5 7.8; 512^2 4.7 4.7 5.6 8.1; 1024^2
+    // - - 6.9 9.2; 32^3 4.3 4.7 5.7 10.2; 64^3 6.6 5.6 6.4 11.2), except that
+    // a grid which fits one block needs no meeting across the chip.  That is
+    // worth up to 4 cells, not 8 (CG, Chebyshev, Jacobi: 64^2, 4 cells in one
+    // block 3.7 1.3 2.6, 1 cell in four 3.4 1.7 3.0; 64 x 128, 8 cells in one
+    // 5.8 2.6 5.0, 1 cell in eight 3.6 2.1 3.2).
     double cost = 1e30;
     for (int k = 1; k <= 8; k *= 2) {
         for (int lxs = 6; lxs >= 4; --lxs) {
@@ -1181,7 +1184,7 @@ Plan plan(int dims, int x, int y, int z, int hd)
             p.ty = (int)tl_cdiv(ny, dims == 2 ? ry * k : ry);
             p.tz = dims == 3 ? (int)tl_cdiv(nz, k) : 1;
             if ((long)p.tx * p.ty * p.tz > most || plan_lds(p) > kMaxLds) continue;
-            const double c = k + (p.blocks() > 1 ? 8.0 : 0.0) + p.blocks() * 1e-3;
+            const double c = k + (p.blocks() > 1 ? 5.0 : 0.0) + p.blocks() * 1e-3;
             if (c < cost) {
                 cost = c;
                 best = p;

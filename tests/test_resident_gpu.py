@@ -46,8 +46,11 @@ CHIP_LOOPS = ("tl_chip_cg", "tl_chip_cheby", "tl_chip_jacobi")
      ["tlhip3d_cheby_solver_iterate"]),
     (tdeck.cuboid_3d(12, 1, solver=tdeck.JACOBI, eps=1e-8, max_iters=300),
      ["tlhip3d_jacobi_solver_iterate"]),
+    # 8192 cells, which one block could hold with 8 cells per thread
+    (tdeck.cuboid_3d(32, 1, solver=tdeck.JACOBI, max_iters=60).replace("z_cells = 32", "z_cells = 8"),
+     ["tlhip3d_jacobi_solver_iterate"]),
 ], ids=["2d-cg", "2d-cg-odd", "2d-cheby", "2d-cheby-odd", "2d-jacobi", "3d-cg", "3d-cheby",
-        "3d-jacobi"])
+        "3d-jacobi", "3d-jacobi-flat"])
 def test_loops_run_where_they_should(hip, loops, text, entries):
     """The timer's launch counts: the on-chip loops alone, or none of them and
     the passes that larger grids run."""
