@@ -17,7 +17,8 @@ namespace pass {
 enum : int { kPQ, kQQ, kRQ, kRR };
 
 // Whether the r.r after an iteration can be predicted: not where it falls
-// below 1% of the one before, as the terms of the prediction then cancel.
+// below 1% of the one before, as the terms of the prediction then cancel (the
+// prediction's error above that line is in tl_chip.hip).
 __host__ __device__ inline bool predictable(double next, double rr)
 {
     return !(next < 0.01 * rr);

@@ -3,9 +3,10 @@
 //
 // A block of 1024 threads owns a tile of up to 8192 cells and at most one
 // block runs per CU, so up to 2.1 million cells stay on the chip for the
-// whole loop: r, A p and the coefficients of a thread's cells in registers,
-// p (with a ring of the neighbours' cells) and kx in LDS.  u is read and
-// written by its own thread only and stays in the CU's cache path.
+// whole loop: r, A p and all but one of the coefficients of a thread's cells
+// in registers, p (with a ring of the neighbours' cells) and the coefficient
+// left (kx, in 3D ky) in LDS.  CG's u stays in memory, read and written by its
+// own thread only; so does Chebyshev's and Jacobi's u0 with 8 cells a thread.
 //
 // Blocks meet once per iteration.  CG has two dot products with a data
 // dependence (alpha = r.r / p.Ap, then beta from the new r.r); here all of
@@ -16,11 +17,15 @@
 //     r'.r' is predicted as r.r - 2 alpha r.q + alpha^2 q.q   (for beta),
 //     r.r is summed from the r in hand                        (for alpha,
 //                                        the stop test and the logs).
-// beta differs from the two-sum form by a few rounding errors; alpha and
-// every vector update are the reference's expressions.  Where the residual
-// falls so far in one iteration that the prediction cancels (below 1% of
-// r.r: its error could pass 1e-13), the blocks meet again and sum the new
-// r.r, as the two-sum form does.
+// alpha and every vector update are the reference's expressions; beta carries
+// more rounding error than the ratio of two sums, as its terms cancel: against
+// the sum of the same r in extended precision (medians) 2e-16 where an
+// iteration leaves half of r.r, 2e-15 where it leaves a tenth, 1e-14 at a
+// fiftieth (largest seen 3e-14), where the sum itself is off by 1e-16.  alpha
+// comes from the real r.r, so nothing of it accumulates, and solutions are as
+// far from an exact solve as with two sums.  Where the residual falls further
+// in one iteration (below 1% of r.r, from where the error could pass 1e-13),
+// the blocks meet again and sum the new r.r, as the two-sum form does.
 //
 // The same meeting hands the tile's outer cells of q to the neighbours: each
 // block also keeps r and p of its ring and updates them with that q, so the
@@ -28,9 +33,10 @@
 //
 // What bounds an iteration is the meeting: a block's sums reach the others in
 // about 1 us and are read back in another, beside 0.3 to 3 us of arithmetic
-// (1 to 8 cells per thread).  512^2 (K = 1) 4.4 us, 1024^2 (K = 4) 6.6, 128^3
-// (K = 8) 21; launch by launch they took 57, 76 and 63 us.  Chebyshev and
-// Jacobi, 1001 x 777: 4.9 us an iteration, 512^2: 4.4 us a sweep (25 and 13).
+// (1 to 4 cells per thread).  512^2 (K = 1) 4.6 us, 1024^2 (K = 4) 6.7; 128^3
+// (K = 8) 19, most of which the meeting and the arithmetic do not account for.
+// Launch by launch they took 57, 76 and 63 us.  Chebyshev and Jacobi, 1001 x
+// 777: 4.9 us an iteration, 512^2: 4.3 us a sweep (25 and 13).
 //
 // Coherence: everything blocks exchange (q of outer cells, the sums) goes
 // through agent-scope atomic loads and stores, which the XCDs' L2s do not
@@ -692,7 +698,8 @@ __global__ void __launch_bounds__(kThreads) k_chip_cg(CgArgs A)
         double* xb = A.xbuf + (size_t)(n & 1) * tl.xall;
         if (nb > 1) tl.hand_over(q, xb);
         const bool go_on = n < A.count;
-        // with few cells per thread, u is on its way while the blocks meet
+        // with few cells per thread, u is loaded ahead of the meeting (whose
+        // drain it shares: the loads are back before the sums are published)
         constexpr bool kEarlyU = K <= 2;
         double u[kEarlyU ? K : 1];
         if constexpr (kEarlyU) {

@@ -255,8 +255,10 @@ def test_graph_replays_match_eager(hip, dims, text):
     """Small grids can replay pairs of resident iterations from a HIP
     graph (tlhip_set_graphs; off by default); otherwise the same iterations
     are enqueued launch by launch.  Every report, u, energy, r and the summary
-    must be the same bits; each solve replays the graph hundreds of times
-    with the host's waits and the loop's own eager launches in between."""
+    must be the same bits; each solve that runs launch by launch replays the
+    graph dozens to hundreds of times with the host's waits and the loop's own
+    eager launches in between (on the chip only PPCG's outer loop has any to
+    replay)."""
     runs = []
     for on in (0, 1):
         hip.tlhip_set_graphs(on)
