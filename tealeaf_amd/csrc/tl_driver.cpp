@@ -14,7 +14,9 @@
 // device-resident (tl_loop.h): alpha, beta, the Jacobi error and the stopping rule are
 // evaluated on the device, the host enqueues iterations ahead and reads one
 // small report per iteration, and the results are those of the host-driven
-// loop bit for bit (tlhip_set_resident(0) selects that loop).
+// loop bit for bit (tlhip_set_resident(0) selects that loop).  CG, Chebyshev
+// and Jacobi loops of grids that fit the chip run many iterations to a launch
+// (tl_chip.h), host-driven one.
 #include <cfloat>
 #include <cmath>
 #include <cstdlib>
@@ -286,9 +288,10 @@ struct tlhip_problem {
     // 0.232 against 0.217 ms per pass).
     bool can_defer_p() const { return g_cg_fusion && dims == 2 && x % 2 == 0 && p_alt; }
 
-    // 2D CG steps (deferred calc_p, halo depth >= 2) run as the cond pair:
-    // calc_pw reads cg_init's conductivity (cond) in place of kx and ky and
-    // keeps w in registers; calc_ur forms w = A p again from p and cond.
+    // 2D CG steps (deferred calc_p, halo depth >= 2) that run neither on the
+    // chip nor as one pass run as the cond pair: calc_pw reads cg_init's
+    // conductivity (cond) in place of kx and ky and keeps w in registers;
+    // calc_ur forms w = A p again from p and cond.
     // u, r and p are the reference's values; rrn is summed in another order.
     // PPCG's calc_pw, whose w the fused inner loop reads, reads cond too and
     // stores w (bit for bit the kx/ky pass).
@@ -298,7 +301,7 @@ struct tlhip_problem {
                (s.coefficient == 1 || s.coefficient == 2);
     }
 
-    // 3D: the CG steps as the 3D cond pair, calc_p deferred into the next
+    // 3D: the CG steps off the chip as the 3D cond pair, calc_p deferred into the next
     // calc_pw (the pending calc_p applied as calc_p + halo update before
     // any other reader of p: PPCG's calc_w, Chebyshev's start).
     bool cond3_ok() const
@@ -1697,12 +1700,6 @@ struct tlhip_problem {
         return 0;
     }
 
-    // The loop of jacobi_driver with jacobi_body's iterations enqueued ahead
-    // of the host.  u_alt starts as a copy of u: sweeps write the interior
-    // and halo updates depth 1 only, so the deeper halo of both buffers stays
-    // the same and u ends as the host-driven loop leaves it.  r is then made
-    // what the host-driven loop leaves: the last sweep's input, with the
-    // residual in its interior when that iteration computed one.
     // Jacobi iterations of grids that fit the chip, many to a launch.  Not in
     // 3D with 8 cells per thread: the sweep's division leaves too few
     // registers (128^3: 46 us a sweep against 24 us with the sweep's own
@@ -1732,6 +1729,12 @@ struct tlhip_problem {
         return 0;
     }
 
+    // The loop of jacobi_driver with jacobi_body's iterations enqueued ahead
+    // of the host.  u_alt starts as a copy of u: sweeps write the interior
+    // and halo updates depth 1 only, so the deeper halo of both buffers stays
+    // the same and u ends as the host-driven loop leaves it.  r is then made
+    // what the host-driven loop leaves: the last sweep's input, with the
+    // residual in its interior when that iteration computed one.
     int jacobi_resident(double* error)
     {
         if (chip_jacobi()) {
